@@ -2,14 +2,15 @@
 // operands, exact int32 accumulation and the i64 requant of golden.py:316-342
 // (NUMERICS.md "GEMM").
 //
-// Two kernels:
-//  * linear_gemv: M <= 16 rows per z-block (decode GEMV, prefill chunks).  One workgroup
+// Three kernels:
+//  * linear_gemv: M <= 16 rows per z-block (decode GEMV, prefill chunks, short prompts).  One workgroup
 //    per 16-column tile; its waves split the K range and each computes a 16(M) x 16(N)
 //    partial tile with v_mfma_i32_16x16x64_i8 (A rows beyond M are zeros supplied in
 //    registers); the partials are summed in LDS.  W [N][K] row-major is streamed once
 //    with 16-byte loads, four K steps in flight per wave.  Integer addition is
 //    associative, so the split never changes a result.
-//  * linear_tiled: M > 16.  128x256 (or 128x128) x 64 block tiles, four waves in 2x2,
+//  * linear_mfma: M > 16, K % 64 == 0.  MFMA tiles over an LDS ring (below).
+//  * linear_tiled: M > 16, other K.  128x256 (or 128x128) x 64 block tiles, four waves in 2x2,
 //    each wave 64x128 (64x64) with v_mfma_i32_32x32x32_i8; A and W double-buffered in LDS.
 //    Blocks are numbered XCD-major so the blocks that share a W panel run on one
 //    XCD and share its L2.
@@ -463,7 +464,7 @@ __device__ __forceinline__ int32_t requant_col(int32_t acc, const ColRq& c) {
 __device__ __forceinline__ int32_t clamp32(int32_t v, int32_t lo, int32_t hi) { return min(max(v, lo), hi); }
 
 // ---------------------------------------------------------------------------------------
-// Large GEMM (M >= 128, K % 64 == 0): GM x GN block tile (256 x 256 with 8 waves, 128 x 128 or
+// Large GEMM (M > 16, K % 64 == 0): GM x GN block tile (256 x 256 with 8 waves, 128 x 128 or
 // 64 x 128 with 4) over K tiles of KT bytes (128 where K allows it, else 64) in an NS-stage LDS ring
 // fed by direct global->LDS loads (global_load_lds_dwordx4)
 // ---------------------------------------------------------------------------------------
@@ -1592,11 +1593,21 @@ template <int EPI, bool OUT8>
 static int launch_linear(LinearArgs& p, void* ws, hipStream_t stream, const NormQuant* norm = nullptr,
                          bool* norm_done = nullptr) {
   const bool aligned = (p.K % 16 == 0) && (p.lda % 16 == 0) && ((uintptr_t)p.A % 16 == 0) && ((uintptr_t)p.W % 16 == 0);
-  if (p.M >= 128 && p.K % 64 == 0 && aligned) {
+  // More than 16 rows: the 16-row kernel over blocks of 16 rows (blockIdx.z) while re-reading W once
+  // per block stays cheap -- every load of a workgroup is requested at entry, so it is one memory
+  // round trip where an LDS ring is one per few K tiles.  Measured (us, 16-row blocks / MFMA tiles):
+  // 64 x 576 x 576 3.3 / 5.6, 64 x 3072 x 1024 5.5 / 7.8, 256 x 896 x 896 5.8 / 6.2, 400 x 576 x 576
+  // 3.9 / 6.0 (ceil(M/16) N K at most 16 MiB), against 400 x 896 x 896 7.4 / 6.5, 64 x 896 x 4864
+  // 7.0 / 6.1 (17 MB and more), 32 x 4864 x 896 9.7 / 8.7 (K past 3072: long serial chains per wave).
+  // Rows that are normalised next (norm) keep the MFMA tiles where those split K (from K = 1024 on):
+  // their finishing launch normalises too, which saves a launch.
+  const bool blocks16 = p.M > 16 && p.M <= 1024 && aligned && p.K <= 3072 && (!norm || p.K < 1024) &&
+                        ceil_div(p.M, 16) * (int64_t)p.N * p.K <= (16ll << 20);
+  if (p.M > 16 && p.K % 64 == 0 && aligned && !blocks16) {
     if (p.K % 128 == 0) return launch_mfma_shape<EPI, OUT8, 128>(p, ws, stream, norm, norm_done);
     return launch_mfma_shape<EPI, OUT8, 64>(p, ws, stream, norm, norm_done);
   }
-  if (p.M > 16 && aligned) {
+  if (p.M > 16 && aligned && !blocks16) {
     // 128x256 block tiles when they still fill the chip, else 128x128
     const int mblocks = (int)ceil_div(p.M, 128);
     const int nb256 = (int)ceil_div(p.N, 256), nb128 = (int)ceil_div(p.N, 128);

@@ -270,6 +270,23 @@ def test_gate_up_equals_the_three_ops(M, K, N, pad, par):
         assert np.array_equal(fq2.cpu().numpy(), got[2])
 
 
+@pytest.mark.parametrize("epilogue,out_i8", [("none", True), ("resadd", False), ("silu", False), ("mul", False)])
+@pytest.mark.parametrize("M,K,N", [(17, 576, 576), (33, 592, 100), (127, 64, 20), (1024, 576, 460), (1025, 576, 460),
+                                   (64, 3072, 1024), (64, 3136, 200), (17, 4864, 896), (65, 896, 4864), (100, 592, 3000)])
+def test_short_prompt_rows(M, K, N, epilogue, out_i8):
+    """17 rows and more: the 16-row blocks (up to 1024 rows, K <= 3072, ceil(M/16) N K <= 16 MiB) with a
+    partial last block, ragged N and K % 64 != 0, and the shapes just past each limit, which take the
+    MFMA tiles (fewer rows than a tile) or, for K % 64 != 0, the 128-row tiles."""
+    rng = np.random.default_rng(M + K + N + len(epilogue))
+    a, w, rq = _operands(rng, M, K, N, out_i8=out_i8)
+    bias = rng.integers(-3000, 3000, N)
+    aux = rng.integers(-32768, 32768, (M, N)) if epilogue in ("resadd", "mul") else None
+    silu = {"Mi": 1 << 30, "Si": 30, "sh_out": 16} if epilogue == "silu" else None
+    shift = 11 if epilogue == "mul" else 0
+    got = gpu_linear(a, w, rq, bias=bias, out_i8=out_i8, epilogue=epilogue, aux=aux, aux_shift=shift, silu=silu)
+    assert np.array_equal(got, O.linear_c(a, w, rq, bias, out_i8, epilogue, aux, shift, silu))
+
+
 @pytest.mark.parametrize("M,K,N", [(512, 4864, 896), (300, 2048, 576), (300, 896, 896), (40, 896, 896), (16, 896, 896),
                                    (16, 4864, 896), (5, 2048, 576), (2, 896, 1024), (512, 896, 896), (256, 1024, 576),
                                    (128, 896, 1024)])
