@@ -47,6 +47,7 @@ struct AttnArgs {
   int32_t* zero;
   int wo_N, zero_n;
   int span;  // dimension-slice launches of one row: XCDs per GQA group (0: one, the grid below)
+  int pslots;  // attention_tiled: tiles per wave whose probabilities are kept in LDS
 };
 
 // clear n int32 values from one workgroup (16-byte aligned)
@@ -438,9 +439,9 @@ __global__ __launch_bounds__(ATTN_THREADS) void attention_rowhead(AttnArgs p) {
 // attention_tiled: M >= 2 rows at consecutive positions pos.. (prefill, chunked prefill)
 // ---------------------------------------------------------------------------------------
 // One workgroup per (block of 16 query rows, query head); its waves split the 64-key tiles of the
-// block's context.  Each of the three reductions is one pass over the tiles, and every pass
-// recomputes the tile's scores with v_mfma_i32_16x16x64_i8 (cheap next to a round trip of the
-// scores through LDS):
+// block's context.  Each of the three reductions is one pass over the tiles; the first two compute a
+// tile's scores with v_mfma_i32_16x16x64_i8 (cheap next to a round trip of 32-bit scores through
+// LDS), the third reads the 16-bit probabilities the second kept:
 //   S^T = K . Q^T : A = 16 key rows, B = the 16 query rows, so lane (lg = lane / 16, lr = lane % 16)
 //                   holds query row lr's scores of keys 16j + 4lg + r (subtile j, register r);
 //   O = P . V     : A = P with row lr and byte 4j + r <-> key 16j + 4lg + r -- exactly the score
@@ -448,8 +449,8 @@ __global__ __launch_bounds__(ATTN_THREADS) void attention_rowhead(AttnArgs p) {
 //                   order, made by multiplying 16-key blocks of V (as A) by 0/1 selection matrices:
 //                   C[key][n] = V[key][16e + n], which lands key 16b + 4lg + r, column 16e + lr in
 //                   lane (lg, lr) register r.
-// The probabilities pn < 2^15 enter the int8 MFMA as base-128 digits (pn = d0 + 128 d1 + 16384 d2,
-// each digit in [0, 127]), so O = O0 + 128 O1 + 16384 O2 is the exact integer sum.  The operand
+// The probabilities pn < 2^15 enter the int8 MFMA as signed base-256 digits (pn = d0 + 256 d1), so
+// O = O0 + 256 O1 is the exact integer sum.  The operand
 // byte order inside a lane (which K index a byte feeds) is the same for A and B, so neither
 // product depends on it.  Keys at or past a row's T get probability 0; keys past the block's last
 // row read zeros.
@@ -489,14 +490,36 @@ __device__ __forceinline__ uint32_t prob_lds(int32_t x, const ProbParams& q, con
   return ((uint32_t)ei[zi >> 8] * (uint32_t)ef[zi & 255] + 32768u) >> 16;
 }
 
+// The rounded LUT product of every exponent index (golden.py:170-172): entry z < 4096 is
+// (kExpI[z >> 8] * kExpF[z & 255] + 32768) >> 16, entries from 4096 on are 0 -- one LDS read per
+// probability instead of two reads and a multiply, and no range check (the index is clamped to 4096).
+struct ExpTable {
+  uint16_t v[4104];
+};
+constexpr ExpTable make_exp_table() {
+  ExpTable t{};
+  for (int z = 0; z < 4096; ++z) t.v[z] = (uint16_t)(((uint32_t)kExpI[z >> 8] * (uint32_t)kExpF[z & 255] + 32768u) >> 16);
+  return t;
+}
+__constant__ constexpr ExpTable kExpT = make_exp_table();
+constexpr int EXPT_CHUNKS = sizeof(ExpTable) / 16;  // 513 16-byte chunks
+
 // MINW: waves per SIMD the register budget must allow.  4 (at most 128 VGPRs) for launches of more
-// waves than fit three to a SIMD: one batched prefill of 16 x 512 rows, 76.9 vs 82.7 us per layer;
-// a single prompt's few workgroups all fit anyway and run faster without the cap (10.16 vs 10.56 us).
+// waves than fit three to a SIMD; a single prompt's few workgroups all fit anyway.
+//
+// What bounds it: VALU work per score (a 16-row block of 1531 keys: 24 tiles x 16 scores per lane),
+// so every per-score step is the fewest full-rate instructions: one 64-bit multiply-add, shift and
+// clamp to the table index, one LDS read, and in the value pass one multiply-add, one funnel shift
+// and half a byte pick per digit.  Tiles entirely inside every row's context skip the masks.  The
+// probabilities of a tile are kept -- packed 16-bit, in registers for the first SC tiles of a wave
+// and in LDS (`pslots` tiles per wave) for the next -- so the value pass computes no score again.
+// Measured against recomputing them with two LUT reads and 64-bit shifts per score: see the dispatch.
 template <int D, int MINW = 1>
 __global__ __launch_bounds__(64 * AttnTileCfg<D>::MAXW, MINW) void attention_tiled(AttnArgs p) {
   using C = AttnTileCfg<D>;
   constexpr int DK = C::DK, DB = C::DB, SC = C::SC;
-  __shared__ uint32_t lut32[LUT_DW];
+  extern __shared__ __attribute__((aligned(16))) v4i pbuf[];  // [pslots][waves][2][64] packed probabilities
+  __shared__ __attribute__((aligned(16))) uint16_t tab[EXPT_CHUNKS * 8];
   __shared__ int32_t red[C::MAXW][AT_ROWS];
   __shared__ int32_t osum[AT_ROWS][D];
   // With Hkv a multiple of 8, GQA group g runs on XCD g % 8 (workgroup b is dispatched to XCD
@@ -511,7 +534,8 @@ __global__ __launch_bounds__(64 * AttnTileCfg<D>::MAXW, MINW) void attention_til
     h = (int)blockIdx.x;
   }
   const int g = h / G;
-  const int m0 = blockIdx.y * AT_ROWS;
+  // the last rows see the most keys: their workgroups are dispatched first
+  const int m0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * AT_ROWS;
   const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
   const int nw = blockDim.x >> 6;
   const int lr = lane & 15, lg = lane >> 4;
@@ -527,6 +551,8 @@ __global__ __launch_bounds__(64 * AttnTileCfg<D>::MAXW, MINW) void attention_til
   const int ntiles = (Tb + 63) >> 6;
   const int m = m0 + lr;  // this lane's query row
   const int tlim = m < p.M ? min(pos + m + 1, (int)p.max_seq) : 0;
+  // tiles whose 64 keys every one of the block's 16 rows sees
+  const int nfull = m0 + AT_ROWS <= p.M ? max(min(pos + m0 + 1, (int)p.max_seq), 0) >> 6 : 0;
   const int8_t* kbase = p.kc + slot + (int64_t)g * p.max_seq * D;
   const int8_t* vbase = p.vc + slot + (int64_t)g * p.max_seq * D;
   const Rsrc kr = rsrc(kbase, (int64_t)Tb * D), vr = rsrc(vbase, (int64_t)Tb * D);
@@ -538,27 +564,9 @@ __global__ __launch_bounds__(64 * AttnTileCfg<D>::MAXW, MINW) void attention_til
     for (int c = 0; c < DK; ++c)
       qf[c] = ld16(qr, (m < p.M && 64 * c + 16 * lg < D) ? (uint32_t)(lr * p.ldq + 64 * c + 16 * lg) : LD_OOB);
   }
-  // the LUT words (words tid, tid + blockDim.x, ..., at least 64 threads; stored to LDS once the tile
-  // loads below are issued, so the two round trips overlap)
-  constexpr int LUTW = (LUT_DW + 63) / 64;
-  uint32_t lutw[LUTW];
-  {
-    const Rsrc ir = rsrc(kExpI, sizeof(kExpI)), fr = rsrc(kExpF, sizeof(kExpF));
-#pragma unroll
-    for (int i = 0; i < LUTW; ++i) {
-      const int idx = tid + i * (int)blockDim.x;
-      lutw[i] = (uint32_t)ld4(ir, idx < 8 ? 4 * idx : LD_OOB) | (uint32_t)ld4(fr, idx >= 8 && idx < LUT_DW ? 4 * (idx - 8) : LD_OOB);
-    }
-  }
   // K (or V) fragment of 16-key block j of tile kt: key kt*64 + 16j + lr, bytes [64c + 16lg, +16)
   auto frag_off = [&](int kt, int j, int c) -> uint32_t {
     return 64 * c + 16 * lg < D ? (uint32_t)((kt * 64 + 16 * j + lr) * D + 64 * c + 16 * lg) : LD_OOB;
-  };
-  auto kfrags = [&](int kt, v4i (&kf)[4][DK]) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int c = 0; c < DK; ++c) kf[j][c] = ld16(kr, frag_off(kt, j, c));
   };
   auto score_mfmas = [&](const v4i (&kf)[4][DK], v4i (&st)[4]) {
 #pragma unroll
@@ -570,20 +578,22 @@ __global__ __launch_bounds__(64 * AttnTileCfg<D>::MAXW, MINW) void attention_til
   };
   auto scores = [&](int kt, v4i (&st)[4]) {
     v4i kf[4][DK];
-    kfrags(kt, kf);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int c = 0; c < DK; ++c) kf[j][c] = ld16(kr, frag_off(kt, j, c));
     score_mfmas(kf, st);
   };
   // key of subtile j, register r of tile kt in this lane
   auto key = [&](int kt, int j, int r) { return kt * 64 + 16 * j + 4 * lg + r; };
 
-  // Tiles wave + it * nw (it < SC) keep their scores, later their probabilities, in registers
-  // across the three passes; further tiles are recomputed in each pass.
+  // Tiles wave + it * nw (it < SC) keep their scores, later their probabilities, in registers.
   v4i cache[SC][4];
   // values of the cached tiles, requested with their keys (used in pass 3)
   v4i vcache[SC][4][DK];
 
-  // pass 1: row maxima.  The cached tiles' keys and values are requested first, then the LUT and
-  // the output sums are staged in LDS (visible after the first barrier).
+  // pass 1: row maxima.  The cached tiles' keys and values are requested first, then the exponential
+  // table and the output sums are staged in LDS (visible after the first barrier).
   int32_t vmax = INT32_MIN;
   v4i kfc[SC][4][DK];
 #pragma unroll
@@ -598,32 +608,44 @@ __global__ __launch_bounds__(64 * AttnTileCfg<D>::MAXW, MINW) void attention_til
 #pragma unroll
       for (int c = 0; c < DK; ++c) vcache[it][j][c] = ld16(vr, kt < ntiles ? frag_off(kt, j, c) : LD_OOB);
   }
+  {
+    const Rsrc tr = rsrc(kExpT.v, sizeof(ExpTable));
+    for (int c = tid; c < EXPT_CHUNKS; c += 4 * (int)blockDim.x) {  // four chunks in flight per thread
+      v4i w[4];
 #pragma unroll
-  for (int i = 0; i < LUTW; ++i) {
-    const int idx = tid + i * (int)blockDim.x;
-    if (idx < LUT_DW) lut32[idx] = lutw[i];
+      for (int u = 0; u < 4; ++u) w[u] = ld16(tr, (uint32_t)(16 * (c + u * (int)blockDim.x)));
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (c + u * (int)blockDim.x < EXPT_CHUNKS) reinterpret_cast<v4i*>(tab)[c + u * (int)blockDim.x] = w[u];
+    }
   }
   for (int idx = tid; idx < AT_ROWS * D; idx += blockDim.x) (&osum[0][0])[idx] = 0;
+  auto tile_max = [&](int kt, const v4i (&st)[4]) {
+    if (kt < nfull) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) vmax = max(vmax, st[j][r]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (key(kt, j, r) < tlim) vmax = max(vmax, st[j][r]);
+    }
+  };
 #pragma unroll
   for (int it = 0; it < SC; ++it) {
     const int kt = wave + it * nw;
     if (kt < ntiles) {
       score_mfmas(kfc[it], cache[it]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (key(kt, j, r) < tlim) vmax = max(vmax, cache[it][j][r]);
+      tile_max(kt, cache[it]);
     }
   }
   for (int kt = wave + SC * nw; kt < ntiles; kt += nw) {
     v4i st[4];
     scores(kt, st);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (key(kt, j, r) < tlim) vmax = max(vmax, st[j][r]);
+    tile_max(kt, st);
   }
   vmax = max(vmax, __shfl_xor(vmax, 16));
   vmax = max(vmax, __shfl_xor(vmax, 32));
@@ -633,53 +655,66 @@ __global__ __launch_bounds__(64 * AttnTileCfg<D>::MAXW, MINW) void attention_til
   for (int w = 1; w < nw; ++w) mx = max(mx, red[w][lr]);
   __syncthreads();
 
-  // pass 2: sums of the LUT exponentials (cached tiles keep p in place of s)
-  const uint16_t* ei = reinterpret_cast<const uint16_t*>(lut32);
-  const uint16_t* ef = ei + 16;
-  ProbParams pq;
-  pq.Ms = (uint32_t)p.Ms;
-  pq.Ss = p.Ss;
-  pq.zc = p.Ss > 0 ? 1ull << (p.Ss - 1) : 0ull;
-  // a tile's 16 scores -> probabilities in place (0 at or past the row's T), returning their sum:
-  // branch-free, all 32 LUT reads issued before the first is used
-  auto tile_probs = [&](int kt, v4i (&st)[4]) -> uint32_t {
-    uint32_t zi[16], lo[16], hi[16];
-    bool ok[16];
+  // pass 2: the LUT exponentials and their sums.  z = rshr((mx - s) Ms, Ss) = ((mx - s) Ms + 2^(Ss-1))
+  // >> Ss (mx - s < 2^24, Ms < 2^32); with Ms < 2^31 and Ss >= 32 it is the high word of the signed
+  // multiply-add (mx Ms + 2^(Ss-1)) - s Ms shifted right by Ss - 32 (below 2^63 for every Ss).
+  const uint32_t Ms = (uint32_t)p.Ms;
+  const uint64_t zc = p.Ss > 0 ? 1ull << (p.Ss - 1) : 0ull;
+  const bool zfast = p.Ms < (1ll << 31) && p.Ss >= 32;
+  const int32_t nMs = (int32_t)(0u - Ms);
+  const int zs = p.Ss - 32;
+  int64_t zrow = (int64_t)mx * (int64_t)Ms + (int64_t)zc;
+  __asm__ volatile("" : "+v"(zrow));  // opaque: keeps one v_mad_i64_i32 per score
+  // a tile's 16 scores -> packed probabilities (0 at or past the row's T), returning their sum
+  auto tile_probs = [&](int kt, const v4i (&st)[4], uint32_t (&pk)[8]) -> uint32_t {
+    uint32_t zi[16];
+    if (zfast) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const uint64_t z = ((uint64_t)(uint32_t)(mx - st[j][r]) * pq.Ms + pq.zc) >> pq.Ss;
-        ok[4 * j + r] = key(kt, j, r) < tlim && z < 4096;
-        zi[4 * j + r] = ok[4 * j + r] ? (uint32_t)z : 0u;
+      for (int k = 0; k < 16; ++k) {
+        const int32_t hi = (int32_t)(((int64_t)st[k >> 2][k & 3] * nMs + zrow) >> 32);
+        zi[k] = (uint32_t)min(hi >> zs, 4096);
       }
+    } else {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      hi[k] = ei[zi[k] >> 8];
-      lo[k] = ef[zi[k] & 255];
+      for (int k = 0; k < 16; ++k) {
+        const uint64_t z = ((uint64_t)(uint32_t)(mx - st[k >> 2][k & 3]) * Ms + zc) >> p.Ss;
+        zi[k] = z < 4096 ? (uint32_t)z : 4096u;
+      }
     }
+    if (kt >= nfull) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) zi[k] = key(kt, k >> 2, k & 3) < tlim ? zi[k] : 4096u;
+    }
+    uint32_t pr[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) pr[k] = tab[zi[k]];
     uint32_t sum = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int k = 4 * j + r;
-        const uint32_t pr = ok[k] ? (hi[k] * lo[k] + 32768u) >> 16 : 0u;
-        st[j][r] = (int32_t)pr;
-        sum += pr;
-      }
+    for (int k = 0; k < 8; ++k) {
+      sum += pr[2 * k] + pr[2 * k + 1];
+      pk[k] = pr[2 * k] | (pr[2 * k + 1] << 16);
+    }
     return sum;
   };
+  uint32_t pk[SC][8];
   uint32_t vsum = 0;
 #pragma unroll
   for (int it = 0; it < SC; ++it) {
     const int kt = wave + it * nw;
-    if (kt < ntiles) vsum += tile_probs(kt, cache[it]);
+    if (kt < ntiles) vsum += tile_probs(kt, cache[it], pk[it]);
   }
-  for (int kt = wave + SC * nw; kt < ntiles; kt += nw) {
+  const int pslots = p.pslots;
+  // this wave's slot of its it-th tile past the cached ones (read back by this wave only)
+  auto pslot = [&](int it) { return pbuf + (it * nw + wave) * 128 + lane; };
+  for (int kt = wave + SC * nw, it = 0; kt < ntiles; kt += nw, ++it) {
     v4i st[4];
+    uint32_t w[8];
     scores(kt, st);
-    vsum += tile_probs(kt, st);
+    vsum += tile_probs(kt, st, w);
+    if (it < pslots) {
+      pslot(it)[0] = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+      pslot(it)[64] = v4i{(int)w[4], (int)w[5], (int)w[6], (int)w[7]};
+    }
   }
   vsum += (uint32_t)__shfl_xor((int)vsum, 16);
   vsum += (uint32_t)__shfl_xor((int)vsum, 32);
@@ -690,8 +725,13 @@ __global__ __launch_bounds__(64 * AttnTileCfg<D>::MAXW, MINW) void attention_til
   const uint32_t inv = 0x80000000u / (total > 1u ? total : 1u);  // 2^31 / total (golden.py:174)
   const uint32_t cap = (1u << p.pb) - 1u;
   const int shp = 31 - p.pb;
-  const uint64_t pc = 1ull << (shp - 1);  // rounding constant of rshr(p * inv, 31 - pb), shp >= 16
-  const bool three = p.pb > 14;           // pn >= 2^14 possible: a third digit
+  uint64_t pc = 1ull << (shp - 1);  // rounding constant of rshr(p * inv, 31 - pb), 16 <= shp <= 23
+  __asm__ volatile("" : "+v"(pc));  // opaque: one v_mad_u64_u32 per probability
+  // The largest probability of a row is that of its maximum, p(z = 0).  Unless some row of the block
+  // is as good as one-hot (then `peak`), no pn reaches cap or 32640 and the clamp and the third
+  // digit below are not needed.
+  const uint32_t top = (uint32_t)(((uint64_t)tab[0] * inv + pc) >> shp);
+  const bool peak = __any(top >= (p.pb == 15 ? 32640u : 256u));
 
   // 0/1 selection matrix e: lane (lg, lr) has byte lr set when lg == e
   v4i sel[4];
@@ -702,24 +742,38 @@ __global__ __launch_bounds__(64 * AttnTileCfg<D>::MAXW, MINW) void attention_til
                  (lr >> 2) == 3 ? (int)bit : 0};
   }
 
-  // pass 3: O = P . V
-  v4i oacc[DB];
+  // pass 3: O = P . V = O0 + 256 O1, the digits' sums accumulated by the MFMAs over all tiles
+  v4i o0[DB], o1[DB];
 #pragma unroll
-  for (int e = 0; e < DB; ++e) oacc[e] = v4i{0, 0, 0, 0};
-  // probabilities (already zero for keys a row does not see) -> base-128 digits -> MFMAs
-  auto pv_tile = [&](const v4i (&pr)[4], const v4i (&vf)[4][DK]) {
+  for (int e = 0; e < DB; ++e) o0[e] = o1[e] = v4i{0, 0, 0, 0};
+  // packed probabilities (zero for keys a row does not see) -> pn -> signed base-256 digits -> MFMAs:
+  // pn = d0 + 256 d1 with d0 = the low byte as a signed value and d1 = (pn + 128) >> 8 <= 127 for pn <
+  // 32640; at or past it (peak) d1 = 127 and d2 = 1 at the same weight
+  auto pv_tile = [&](const uint32_t (&w)[8], const v4i (&vf)[4][DK]) {
     v4i pd[3];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      uint32_t pn[4];
+      uint32_t n[2];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const uint32_t v = (uint32_t)(((uint64_t)(uint32_t)pr[j][r] * inv + pc) >> shp);
-        pn[r] = v < cap ? v : cap;
+      for (int i = 0; i < 2; ++i) {
+        const uint64_t a = (uint64_t)(w[2 * j + i] & 0xFFFFu) * inv + pc, b = (uint64_t)(w[2 * j + i] >> 16) * inv + pc;
+        uint32_t pa = __builtin_amdgcn_alignbit((uint32_t)(a >> 32), (uint32_t)a, shp);
+        uint32_t pb = __builtin_amdgcn_alignbit((uint32_t)(b >> 32), (uint32_t)b, shp);
+        if (peak) {
+          pa = min(pa, cap);
+          pb = min(pb, cap);
+        }
+        n[i] = pa | (pb << 16);
       }
-      pd[0][j] = (int)pack4(pn[0] & 127, pn[1] & 127, pn[2] & 127, pn[3] & 127);
-      pd[1][j] = (int)pack4((pn[0] >> 7) & 127, (pn[1] >> 7) & 127, (pn[2] >> 7) & 127, (pn[3] >> 7) & 127);
-      pd[2][j] = (int)pack4(pn[0] >> 14, pn[1] >> 14, pn[2] >> 14, pn[3] >> 14);
+      pd[0][j] = (int)__builtin_amdgcn_perm(n[1], n[0], 0x06040200u);
+      uint32_t q0 = n[0] + 0x00800080u, q1 = n[1] + 0x00800080u;  // halves stay below 2^16
+      if (peak) {
+        const uint32_t t0 = (q0 >> 15) & 0x00010001u, t1 = (q1 >> 15) & 0x00010001u;
+        q0 -= t0 << 8;
+        q1 -= t1 << 8;
+        pd[2][j] = (int)__builtin_amdgcn_perm(t1, t0, 0x06040200u);
+      }
+      pd[1][j] = (int)__builtin_amdgcn_perm(q1, q0, 0x07050301u);
     }
 #pragma unroll
     for (int e = 0; e < DB; ++e) {
@@ -730,32 +784,40 @@ __global__ __launch_bounds__(64 * AttnTileCfg<D>::MAXW, MINW) void attention_til
         const v4i t = __builtin_amdgcn_mfma_i32_16x16x64_i8(vf[b][c], sel[e & 3], v4i{0, 0, 0, 0}, 0, 0, 0);
         vt[b] = (int)pack4(t[0], t[1], t[2], t[3]);
       }
-      const v4i a0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(pd[0], vt, v4i{0, 0, 0, 0}, 0, 0, 0);
-      const v4i a1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(pd[1], vt, v4i{0, 0, 0, 0}, 0, 0, 0);
-      const v4i a2 = three ? __builtin_amdgcn_mfma_i32_16x16x64_i8(pd[2], vt, v4i{0, 0, 0, 0}, 0, 0, 0) : v4i{0, 0, 0, 0};
-#pragma unroll
-      for (int r = 0; r < 4; ++r) oacc[e][r] += a0[r] + 128 * a1[r] + 16384 * a2[r];
+      o0[e] = __builtin_amdgcn_mfma_i32_16x16x64_i8(pd[0], vt, o0[e], 0, 0, 0);
+      o1[e] = __builtin_amdgcn_mfma_i32_16x16x64_i8(pd[1], vt, o1[e], 0, 0, 0);
+      if (peak) o1[e] = __builtin_amdgcn_mfma_i32_16x16x64_i8(pd[2], vt, o1[e], 0, 0, 0);
     }
   };
 #pragma unroll
   for (int it = 0; it < SC; ++it)
-    if (wave + it * nw < ntiles) pv_tile(cache[it], vcache[it]);
-  for (int kt = wave + SC * nw; kt < ntiles; kt += nw) {
+    if (wave + it * nw < ntiles) pv_tile(pk[it], vcache[it]);
+  for (int kt = wave + SC * nw, it = 0; kt < ntiles; kt += nw, ++it) {
     v4i vf[4][DK];
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
       for (int c = 0; c < DK; ++c) vf[b][c] = ld16(vr, frag_off(kt, b, c));
-    v4i st[4];
-    scores(kt, st);
-    tile_probs(kt, st);
-    pv_tile(st, vf);
+    uint32_t w[8];
+    if (it < pslots) {
+      const v4i a = pslot(it)[0], b = pslot(it)[64];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        w[i] = (uint32_t)a[i];
+        w[4 + i] = (uint32_t)b[i];
+      }
+    } else {
+      v4i st[4];
+      scores(kt, st);
+      tile_probs(kt, st, w);
+    }
+    pv_tile(w, vf);
   }
   // C layout of O: lane (lg, lr) register r = row 4lg + r, column 16e + lr
 #pragma unroll
   for (int e = 0; e < DB; ++e)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) atomicAdd(&osum[4 * lg + r][16 * e + lr], oacc[e][r]);
+    for (int r = 0; r < 4; ++r) atomicAdd(&osum[4 * lg + r][16 * e + lr], o0[e][r] + 256 * o1[e][r]);
   __syncthreads();
   for (int idx = tid; idx < AT_ROWS * D; idx += blockDim.x) {
     const int row = idx / D, d = idx % D;
@@ -1558,16 +1620,16 @@ static int attention_impl(const int8_t* q, int64_t M, int64_t H, int64_t Hkv, in
     while (nw < maxw && nw * 2 <= tiles && (nw * sc < tiles || blocks * nw < 4 * (int64_t)current_cu_count())) nw *= 2;
     dim3 grid((unsigned)H, (unsigned)ceil_div(M, AT_ROWS));
     dim3 block(64 * nw);
-    const bool dense = blocks * nw > 12ll * current_cu_count();  // more waves than three per SIMD
+    // probabilities of the tiles past the cached ones kept in LDS: up to 64 KB, two workgroups per CU
+    const int64_t slots = std::max<int64_t>(0, ceil_div(tiles, nw) - sc);
+    p.pslots = (int)std::min<int64_t>(slots, (64 << 10) / (2048 * nw));
+    const unsigned lds = (unsigned)(p.pslots * nw * 2048);
     switch (D) {
-      case 16: hipLaunchKernelGGL(attention_tiled<16>, grid, block, 0, s, p); break;  // 4 waves/SIMD as they are
-      case 32: hipLaunchKernelGGL(attention_tiled<32>, grid, block, 0, s, p); break;
-      case 64:
-        if (dense) hipLaunchKernelGGL((attention_tiled<64, 4>), grid, block, 0, s, p);
-        else hipLaunchKernelGGL(attention_tiled<64>, grid, block, 0, s, p);
-        break;
-      case 128: hipLaunchKernelGGL(attention_tiled<128>, grid, block, 0, s, p); break;
-      default: hipLaunchKernelGGL(attention_tiled<256>, grid, block, 0, s, p); break;
+      case 16: hipLaunchKernelGGL(attention_tiled<16>, grid, block, lds, s, p); break;
+      case 32: hipLaunchKernelGGL(attention_tiled<32>, grid, block, lds, s, p); break;
+      case 64: hipLaunchKernelGGL(attention_tiled<64>, grid, block, lds, s, p); break;
+      case 128: hipLaunchKernelGGL(attention_tiled<128>, grid, block, lds, s, p); break;
+      default: hipLaunchKernelGGL(attention_tiled<256>, grid, block, lds, s, p); break;
     }
     LLHIP_LAUNCH_CHECK();
     return 0;

@@ -36,7 +36,7 @@ def hip_tables_text() -> str:
     lines = ["// GENERATED by llaccel_amd/luts.py -- do not edit.", ""]
     sig_padded = np.append(sigmoid_lut(), np.uint16(0))
     for name, arr in (("kSig", sig_padded), ("kExpI", exp_int_lut()), ("kExpF", exp_frac_lut())):
-        lines.append(f"static __constant__ uint16_t {name}[{len(arr)}] = {{")
+        lines.append(f"static __constant__ constexpr uint16_t {name}[{len(arr)}] = {{")
         for i in range(0, len(arr), 16):
             lines.append("    " + ", ".join(f"{int(v)}" for v in arr[i:i + 16]) + ",")
         lines.append("};")
