@@ -1611,13 +1611,21 @@ static int attention_impl(const int8_t* q, int64_t M, int64_t H, int64_t Hkv, in
   }
   if (tiled) {
     // waves per workgroup: enough that every wave's tiles stay in registers across the three
-    // passes, more (up to the register-file limit) while the chip would otherwise be idle
+    // passes, more (up to the register-file limit) while the chip would otherwise be idle.  Launches
+    // of at least one workgroup per CU stop at four waves while the rest of their tiles' packed
+    // probabilities take at most 32 KB of LDS (D >= 128, whose registers allow two or three waves
+    // per SIMD in any case: 64 KB): every wave repeats the prologue and the barriers.  Measured, four
+    // / eight waves: 1024 rows of D = 64 16.5 / 18.1 us, 8 x 1024 84.7 / 100 us, 1536 rows of D = 128
+    // 64.8 / 78.0 us, 4 x 512 40.8 / 63.8 us; past the limits 2048 rows of D = 64 48.4 / 41.2 us,
+    // 4096 rows of D = 128 512 / 435 us.
     const int64_t blocks = H * ceil_div(M, AT_ROWS);
     const int maxw = D <= 128 ? AttnTileCfg<128>::MAXW : AttnTileCfg<256>::MAXW;
     const int sc = D <= 64 ? AttnTileCfg<64>::SC : 1;
     const int64_t tiles = ceil_div(tmax, 64);
+    const bool four = blocks >= cus && tiles <= 4 * (sc + (D <= 64 ? 4 : 8));
     int nw = 1;
-    while (nw < maxw && nw * 2 <= tiles && (nw * sc < tiles || blocks * nw < 4 * (int64_t)current_cu_count())) nw *= 2;
+    while (nw < (four ? std::min(maxw, 4) : maxw) && nw * 2 <= tiles && (nw * sc < tiles || blocks * nw < 4 * (int64_t)cus))
+      nw *= 2;
     dim3 grid((unsigned)H, (unsigned)ceil_div(M, AT_ROWS));
     dim3 block(64 * nw);
     // probabilities of the tiles past the cached ones kept in LDS: up to 64 KB, two workgroups per CU

@@ -46,11 +46,15 @@ CASES = [
     (20, 8, 2, 64, 3000, 4096),
     (3, 4, 2, 32, 2500, 3000),
     (1, 2, 1, 16, 2047, 2048),
-    # launches of more waves than fit three to a SIMD (a batched prefill's size; at D = 64 the
-    # register-capped instance of the multi-row kernel)
+    # launches of more waves than fit three to a SIMD (a batched prefill's size)
     (2048, 14, 2, 64, 0, 2048),
     (1024, 8, 2, 16, 0, 1024),
     (1024, 8, 4, 32, 0, 1024),
+    # four waves with more tiles than their registers hold (probabilities in LDS), and eight waves with
+    # more than the LDS holds as well (recomputed in the value pass); a ragged last row block
+    (800, 14, 2, 64, 0, 1024),
+    (602, 16, 8, 128, 0, 640),
+    (250, 16, 8, 128, 3840, 4096),
 ]
 
 
@@ -168,10 +172,11 @@ def test_rows_as_sequences(D, H, Hkv):
 
 
 @pytest.mark.parametrize("M,D", [(16, 64), (1, 64), (40, 128), (5, 256)])
-@pytest.mark.parametrize("regime", ["onehot", "flat", "extreme"])
+@pytest.mark.parametrize("regime", ["onehot", "steep", "flat", "extreme"])
 def test_softmax_regimes(M, D, regime):
-    """Saturating probabilities (one key gets 2^pb - 1, so every base-128 digit of pn is used),
-    a flat softmax (Ms = 0: every p = 65534) and all-(-128) operands (maximal scores)."""
+    """Saturating probabilities (one key gets 2^pb - 1: the clamp and the third digit of pn are used),
+    the same with the largest Ms and the smallest Ss of the 32-bit index form, a flat softmax (Ms = 0:
+    every p = 65534) and all-(-128) operands (maximal scores)."""
     rng = np.random.default_rng(M + D + len(regime))
     H, Hkv, pos, max_seq = 4, 2, 70, 128
     kc = rng.integers(-128, 128, (Hkv, max_seq, D)).astype(np.int8)
@@ -180,6 +185,8 @@ def test_softmax_regimes(M, D, regime):
     Ms, Ss, Mo, So = (1 << 31) + 12345, 20, (1 << 31) - 1, 40
     if regime == "flat":
         Ms = 0
+    elif regime == "steep":
+        Ms, Ss = (1 << 31) - 1, 32
     elif regime == "extreme":
         kc[:] = -128
         vc[:] = -128
