@@ -33,22 +33,26 @@ namespace llhip {
 // RMSNorm + quant prologue (golden.py:124-137, 119-120)
 // ---------------------------------------------------------------------------------------
 
-// Rows and 4-element output units of this wave.  With M < nw several waves share a row: each
+// Rows and 4-element output units of this wave.  With 2 M <= nw several waves share a row: each
 // computes the row's sum of squares (the row is 2 KiB at most) and applies the scale to its own
-// units, so no cross-wave reduction is needed.  With M >= nw wave w takes rows w, w + nw, ...
+// units, so no cross-wave reduction is needed.  Otherwise (full) wave w takes the rows w, w + nw, ...
+// whole, two at a time.
 struct NormMap {
   int m0, step, j, G;  // rows m0, m0 + step, ...; units j*64 + lane + i*G*64
+  bool full;
 };
 
 __device__ __forceinline__ NormMap norm_map(int M) {
-  const int wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int wave = wave_id(), nw = blockDim.x >> 6;
   NormMap r;
-  r.m0 = wave % M;
-  if (M < nw) {
+  r.full = 2 * M > nw;
+  if (!r.full) {
+    r.m0 = wave % M;
     r.step = M;
     r.j = wave / M;
     r.G = (nw - r.m0 + M - 1) / M;
   } else {
+    r.m0 = wave;
     r.step = nw;
     r.j = 0;
     r.G = 1;
@@ -56,16 +60,32 @@ __device__ __forceinline__ NormMap norm_map(int M) {
   return r;
 }
 
-// operands of the wave's first row, loaded at kernel entry
+// operands of the wave's first row (full: first two rows), loaded at kernel entry
 struct NormRegs {
-  v4i xs[2];  // 8-element chunks lane and lane + 64 (sum of squares)
-  v2i xu, gu; // x and gamma of the first output unit
+  v4i xs[2];   // 8-element chunks lane and lane + 64 (sum of squares; full: the whole row)
+  v2i xu, gu;  // x and gamma of the first output unit
+  v4i x1[2];   // full: the second row's chunks
+  v4i g[2];    // full: gamma chunks
 };
+
+// the 8-element chunks lane and lane + 64 of the row at byte offset `row`
+__device__ __forceinline__ void norm_row_load(Rsrc xr, uint32_t row, int nch, v4i (&x)[2]) {
+  const int lane = threadIdx.x & 63;
+  x[0] = ld16(xr, lane < nch ? row + 16 * lane : LD_OOB);
+  x[1] = ld16(xr, lane + 64 < nch ? row + 16 * (lane + 64) : LD_OOB);
+}
 
 __device__ __forceinline__ void norm_prefetch(const NormQuant& pr, int M, const NormMap& nm, NormRegs& r) {
   const int lane = threadIdx.x & 63, nch = pr.K >> 3, nu = pr.K >> 2;
   const Rsrc xr = rsrc(pr.x, (int64_t)M * pr.ldx * 2), gr = rsrc(pr.gamma, (int64_t)pr.K * 2);
   const uint32_t row = (uint32_t)(nm.m0 * pr.ldx * 2);
+  if (nm.full) {
+    if (nm.m0 >= M) return;  // this wave has no row
+    norm_row_load(xr, row, nch, r.xs);
+    if (nm.m0 + nm.step < M) norm_row_load(xr, row + (uint32_t)(nm.step * pr.ldx * 2), nch, r.x1);
+    norm_row_load(gr, 0, nch, r.g);
+    return;
+  }
   r.xs[0] = ld16(xr, lane < nch ? row + 16 * lane : LD_OOB);
   r.xs[1] = ld16(xr, lane + 64 < nch ? row + 16 * (lane + 64) : LD_OOB);
   const int u = nm.j * 64 + lane;
@@ -111,12 +131,72 @@ __device__ __forceinline__ void norm_apply_unit(const NormQuant& pr, int m, int 
   }
 }
 
+// One whole row from registers: chunks lane and lane + 64 normalised, quantised and stored.
+__device__ __forceinline__ void norm_apply_row(const NormQuant& pr, int m, uint32_t inv, const v4i (&x)[2],
+                                               const v4i (&g)[2], int8_t* a_lds, int lda, bool write_global) {
+  const int lane = threadIdx.x & 63, nch = pr.K >> 3;
+  const double sy = rms_scale(inv, pr.sh_post), sq = mulshift_scale(pr.Mq, pr.Sq);  // exact forms
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int c = lane + 64 * i;
+    v4i y;
+    v2i q;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int32_t y0 = rms_apply_d(lo16(x[i][j]), lo16(g[i][j]), sy), y1 = rms_apply_d(hi16(x[i][j]), hi16(g[i][j]), sy);
+      y[j] = pack16(y0, y1);
+      const uint32_t w = (uint32_t)(uint8_t)mulshift_small_sat(y0, sq, -128.0, 127.0) |
+                         ((uint32_t)(uint8_t)mulshift_small_sat(y1, sq, -128.0, 127.0) << 8);
+      q[j >> 1] = (j & 1) ? (int)((uint32_t)q[j >> 1] | (w << 16)) : (int)w;
+    }
+    if (c < nch) {
+      *reinterpret_cast<v2i*>(a_lds + m * lda + 8 * c) = q;
+      if (write_global) {
+        if (pr.h_out) *reinterpret_cast<v4i*>(pr.h_out + (int64_t)m * pr.ldx + 8 * c) = y;
+        if (pr.hq_out) *reinterpret_cast<v2i*>(pr.hq_out + (int64_t)m * pr.K + 8 * c) = q;
+      }
+    }
+  }
+}
+
+// Rows m0, m0 + step, ... of this wave, two at a time so that the two rows' serial chains (sum,
+// square root, division) overlap; the first two from the registers loaded at entry, so that nothing
+// but the weights is waited for behind them.  Replaces a launch of its own for M > 1: a decode step
+// of 8 rows, 30 layers of 576, 894 -> 803 us; of 16 rows, 24 layers of 896: attn_in 7.0 + 2.9 us in two
+// launches, 8.8 us in one.
+__device__ __forceinline__ void norm_rows_full(const NormQuant& pr, const NormRegs& r, int M, const NormMap& nm,
+                                               int8_t* a_lds, int lda, bool write_global) {
+  const int nch = pr.K >> 3;
+  const Rsrc xr = rsrc(pr.x, (int64_t)M * pr.ldx * 2);
+  auto rows = [&](int m, const v4i (&x0)[2], const v4i (&x1)[2]) {
+    if (m + nm.step < M) {
+      const uint32_t i0 = norm_row_inv(pr, x0[0], x0[1]), i1 = norm_row_inv(pr, x1[0], x1[1]);
+      norm_apply_row(pr, m, i0, x0, r.g, a_lds, lda, write_global);
+      norm_apply_row(pr, m + nm.step, i1, x1, r.g, a_lds, lda, write_global);
+    } else {
+      norm_apply_row(pr, m, norm_row_inv(pr, x0[0], x0[1]), x0, r.g, a_lds, lda, write_global);
+    }
+  };
+  if (nm.m0 >= M) return;
+  rows(nm.m0, r.xs, r.x1);
+  for (int m = nm.m0 + 2 * nm.step; m < M; m += 2 * nm.step) {
+    v4i a[2], b[2];
+    norm_row_load(xr, (uint32_t)(m * pr.ldx * 2), nch, a);
+    norm_row_load(xr, (uint32_t)((m + nm.step) * pr.ldx * 2), nch, b);  // past row M - 1: zeros
+    rows(m, a, b);
+  }
+}
+
 // The wave's first row and first unit use the registers loaded at entry in straight-line code,
-// so their waits cover those loads only; further rows and units (M > waves, or K > 256 * waves
-// sharing a row) load inside loops.
-__device__ void norm_quant_rows(const NormQuant& pr, const NormRegs& r, int M, const NormMap& nm, int8_t* a_lds,
-                                int lda, bool write_global) {
-  const int lane = threadIdx.x & 63, nch = pr.K >> 3, nu = pr.K >> 2;
+// so their waits cover those loads only; further units (K > 256 * waves sharing a row) load inside
+// loops.
+__device__ __forceinline__ void norm_quant_rows(const NormQuant& pr, const NormRegs& r, int M, const NormMap& nm,
+                                                int8_t* a_lds, int lda, bool write_global) {
+  if (nm.full) {
+    norm_rows_full(pr, r, M, nm, a_lds, lda, write_global);
+    return;
+  }
+  const int lane = threadIdx.x & 63, nu = pr.K >> 2;
   const Rsrc xr = rsrc(pr.x, (int64_t)M * pr.ldx * 2), gr = rsrc(pr.gamma, (int64_t)pr.K * 2);
   const int ustep = nm.G * 64;
   {
@@ -125,17 +205,6 @@ __device__ void norm_quant_rows(const NormQuant& pr, const NormRegs& r, int M, c
     const uint32_t inv = norm_row_inv(pr, r.xs[0], r.xs[1]);
     norm_apply_unit(pr, m, nm.j * 64 + lane, inv, r.xu, r.gu, a_lds, lda, write_global);
     for (int u0 = nm.j * 64 + ustep; u0 < nu; u0 += ustep) {
-      const int u = u0 + lane;
-      const v2i xu = ld8(xr, u < nu ? row + 8 * u : LD_OOB), gu = ld8(gr, u < nu ? 8 * u : LD_OOB);
-      norm_apply_unit(pr, m, u, inv, xu, gu, a_lds, lda, write_global);
-    }
-  }
-  for (int m = nm.m0 + nm.step; m < M; m += nm.step) {
-    const uint32_t row = (uint32_t)(m * pr.ldx * 2);
-    const v4i xs0 = ld16(xr, lane < nch ? row + 16 * lane : LD_OOB);
-    const v4i xs1 = ld16(xr, lane + 64 < nch ? row + 16 * (lane + 64) : LD_OOB);
-    const uint32_t inv = norm_row_inv(pr, xs0, xs1);
-    for (int u0 = nm.j * 64; u0 < nu; u0 += ustep) {
       const int u = u0 + lane;
       const v2i xu = ld8(xr, u < nu ? row + 8 * u : LD_OOB), gu = ld8(gr, u < nu ? 8 * u : LD_OOB);
       norm_apply_unit(pr, m, u, inv, xu, gu, a_lds, lda, write_global);
@@ -992,8 +1061,9 @@ struct NormGemvArgs {
   int ring_cap, vocab;
 };
 
+// (64 VGPRs: four workgroups of eight waves per CU; at 68 the 16-row head took 38.8 us, 34.9 at 64)
 template <int MAXW>
-__global__ __launch_bounds__(64 * MAXW) void norm_gemv_kernel(NormGemvArgs p) {
+__global__ __launch_bounds__(64 * MAXW, 4) void norm_gemv_kernel(NormGemvArgs p) {
   kernarg_warm<sizeof(NormGemvArgs)>();
   extern __shared__ __attribute__((aligned(16))) int8_t dyn[];
   __shared__ v4i red[MAXW][64];
@@ -1303,6 +1373,9 @@ static int mlp_in_args(const llhip_mlp_in_desc* d, MlpInArgs& p, int min_threads
   const int tiles = (int)ceil_div(N, 16);
   if (!w_ok(N, K)) return fail(-EINVAL, "mlp_in: weights above 2 GiB");
   p.KS = pick_ks(tiles, 2, (int)ceil_div(K, 64), FUSED_WAVES);
+  // rows normalised here: a wave takes at most two of them, all loaded at entry, where waves allow it
+  if (M > 1 && !p.pre.prequant)
+    while (4 * p.KS < M && 4 * p.KS <= FUSED_WAVES && 2 * p.KS <= (int)ceil_div(K, 64)) p.KS *= 2;
   while (128 * p.KS < min_threads && 2 * p.KS < FUSED_WAVES) ++p.KS;  // one row unit per thread
   if (128 * p.KS < min_threads) return fail(-EINVAL, "mlp_in: no workgroup shape fits");
   const size_t lds = (size_t)(M * (K + 16));
@@ -1311,9 +1384,21 @@ static int mlp_in_args(const llhip_mlp_in_desc* d, MlpInArgs& p, int min_threads
 }
 
 extern "C" int llhip_mlp_in(const llhip_mlp_in_desc* d, void* stream) {
+  if (!d) return fail(-EINVAL, "mlp_in: null descriptor");
+  // More than 8 rows and more workgroups than CUs (two prologues on some CUs): the rows normalised
+  // once, in a launch of their own.  16 rows of 896, FFN 4864 (304 workgroups): 12.2 us with the rows
+  // normalised in every workgroup against 8.3 + 2.9 us; FFN 1536 (96 workgroups) 12 rows 6.5 against
+  // 6.4 + 2.5 us, and 8 rows of FFN 4864 gain too.
+  llhip_mlp_in_desc dd = *d;
+  const bool apart = !d->pre.prequant && d->M > 8 && d->pre.hq_out && ceil_div(d->N, 16) > current_cu_count();
+  if (apart) dd.pre.prequant = 1;
   MlpInArgs p{};
-  const int rc = mlp_in_args(d, p, 0);
+  const int rc = mlp_in_args(&dd, p, 0);
   if (rc) return rc;
+  if (apart) {
+    const int nrc = llhip_rmsnorm_quant(&d->pre, d->M, stream);
+    if (nrc) return nrc;
+  }
   hipLaunchKernelGGL((mlp_in_kernel<FUSED_WAVES>), dim3((unsigned)ceil_div(p.N, 16)), dim3(128 * p.KS),
                      (size_t)(p.M * (p.K + 16)), (hipStream_t)stream, p);
   LLHIP_LAUNCH_CHECK();

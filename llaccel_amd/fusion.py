@@ -56,9 +56,11 @@ class FusedStep:
             return
         self.fill(self.desc, M, pos, pd)
         m = self.model
-        # several rows: normalise them once (one launch) instead of in every workgroup's prologue
-        self.desc.pre.prequant = int(M > 1)
-        if M > 1:
+        # several rows of the head: normalise them once (one launch) instead of in each of its
+        # thousands of workgroups; the layers' few hundred normalise them in their prologues, while
+        # their weights are on the way
+        self.desc.pre.prequant = int(M > 1 and self.kind == "norm_linear")
+        if self.desc.pre.prequant:
             _lib.call("llhip_rmsnorm_quant", ctypes.byref(self.desc.pre), M, m._stream_handle())
         _lib.call(self.entry, ctypes.byref(self.desc), m._stream_handle())
 

@@ -182,3 +182,40 @@ def test_prefill_batch_other_lengths_run_separately(tmp_path_factory):
     assert calls == [] and [len(r) for r in rows] == [40, 33]
     s = G.GoldenModel(qdir)
     assert np.array_equal(np.asarray(rows[1][32]), np.asarray(s.prefill(prompts[1])[32]))
+
+
+@pytest.mark.parametrize("K,N", [(576, 1536), (896, 4880), (1024, 48), (16, 32)])
+@pytest.mark.parametrize("M", [2, 3, 4, 5, 7, 8, 9, 13, 16])
+def test_rows_normalised_in_the_prologue(M, K, N):
+    """llhip_mlp_in of several rows normalising them in every workgroup (several waves to a row, one
+    wave to one, two or more rows; past 8 rows and one workgroup per CU a launch of its own) writes
+    what llhip_rmsnorm_quant followed by the prequantised form writes."""
+    import ctypes
+
+    from llaccel_amd import _lib
+    from tests.gpu_helpers import ptr, random_rq, stream, torch, up
+
+    t = torch()
+    rng = np.random.default_rng(100 * M + K)
+    x, g = up(rng.integers(-32768, 32768, (M, K)), np.int16), up(rng.integers(-32768, 32768, K), np.int16)
+    wg, wu = (up(rng.integers(-127, 128, (N, K)), np.int8) for _ in range(2))
+    rqg, rqu = (up(random_rq(rng, N, K, False), np.int32) for _ in range(2))
+    outs = []
+    for pre in (0, 1):
+        h, hq = t.zeros((M, K), dtype=t.int16, device="cuda"), t.zeros((M, K), dtype=t.int8, device="cuda")
+        sg, f = (t.zeros((M, N), dtype=t.int16, device="cuda") for _ in range(2))
+        fq = t.zeros((M, N), dtype=t.int8, device="cuda")
+        d = _lib.MlpInDesc()
+        n = d.pre
+        n.x, n.gamma, n.h_out, n.hq_out, n.ldx, n.K = ptr(x), ptr(g), ptr(h), ptr(hq), K, K
+        n.eps_t, n.C, n.sh_post, n.Mq, n.Sq, n.prequant = 999, int(2**24 * K**0.5), 24, 1234567891, 38, pre
+        d.Wg, d.Wu, d.rqg, d.rqu = ptr(wg), ptr(wu), ptr(rqg), ptr(rqu)
+        d.sg_out, d.f_out, d.fq_out = ptr(sg), ptr(f), ptr(fq)
+        d.silu_Mi, d.silu_Si, d.silu_sh, d.mul_sh, d.fq_M, d.fq_S, d.M, d.N = 1 << 30, 30, 16, 11, 1 << 30, 37, M, N
+        if pre:
+            _lib.call("llhip_rmsnorm_quant", ctypes.byref(n), M, stream())
+        _lib.call("llhip_mlp_in", ctypes.byref(d), stream())
+        outs.append([a.cpu().numpy() for a in (h, hq, sg, f, fq)])
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
+    assert np.abs(outs[0][4]).max() > 0
