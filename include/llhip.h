@@ -124,6 +124,12 @@ int llhip_linear(const int8_t* A, int64_t M, int64_t K, int64_t lda, const int8_
                  const int32_t* bias, int epilogue, const int16_t* aux, int64_t ldaux, int64_t aux_shift,
                  int64_t silu_Mi, int64_t silu_Si, int64_t silu_sh, int out_i8, void* out, int64_t ldo, void* ws,
                  void* stream);
+/* golden.py:316-342 + 115-116  the projection and the residual add of an unfused graph's layer: o =
+ * llhip_linear (epilogue none, i16) and out = llhip_vadd(a, o, sh_b), both written, rows of ld = N
+ * values.  One launch for up to 16 rows and for the longer calls that run as blocks of 16 rows. */
+int llhip_linear_add(const int8_t* A, int64_t M, int64_t K, int64_t lda, const int8_t* W, int64_t N, const int32_t* rq,
+                     const int32_t* bias, const int16_t* a, int64_t sh_b, int16_t* o, int16_t* out, int64_t ld, void* ws,
+                     void* stream);
 /* golden.py:316-342 (silu and mul epilogues) + 119-120  the gate and up projections of an MLP over
  * M rows in one launch: sg = silu16(requant16(A . Wg^T + bg)), f = sat16(rshr(requant16(A . Wu^T +
  * bu) * sg, mul_sh)), fq = quant(f), outputs [M][ld] (i16, i16, i8) -- the values of the gate

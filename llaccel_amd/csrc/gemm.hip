@@ -24,7 +24,7 @@ namespace llhip {
 
 typedef int v16i __attribute__((ext_vector_type(16)));
 
-enum Epi : int { EPI_NONE = 0, EPI_RESADD = 1, EPI_SILU = 2, EPI_MUL = 3, EPI_ROPE = 4 };
+enum Epi : int { EPI_NONE = 0, EPI_RESADD = 1, EPI_SILU = 2, EPI_MUL = 3, EPI_ROPE = 4, EPI_ADD = 5 };
 
 
 struct LinearArgs {
@@ -43,6 +43,9 @@ struct LinearArgs {
   int nfast;   // linear_mfma: tiles in N-fastest order (N-block l % nblk), else M-fastest
   int nblk;
   int mgroup;  // M-fastest order within groups of mgroup M-blocks (0: one group of all)
+  // EPI_ADD, the linear and add of an unfused graph (linear_gemv, linear_gemv1): the linear's own
+  // output rows (stride ldo), kept beside the sum; the add's shift of them is aux_shift
+  int16_t* pre;
 };
 
 // M-block and N-block of logical tile l: N-block fastest (nfast), or M-block fastest within groups
@@ -132,7 +135,10 @@ __device__ __forceinline__ void finish_pre(const LinearArgs& p, const EpiOperand
     return;
   }
   int64_t t = sat16(v);
-  if (EPI == EPI_RESADD) t = sat16(t + e.aux[r]);
+  if (EPI == EPI_ADD) {
+    p.pre[(int64_t)m * p.ldo + n] = (int16_t)t;
+    t = sat16(rshr32_any((int32_t)t, p.aux_shift) + e.aux[r]);
+  } else if (EPI == EPI_RESADD) t = sat16(t + e.aux[r]);
   else if (EPI == EPI_SILU) t = silu16(t, p.Mi, p.Si, p.sh);
   else if (EPI == EPI_MUL) t = sat16(rshr(wmul(t, e.aux[r]), p.aux_shift));
   static_cast<int16_t*>(p.out)[(int64_t)m * p.ldo + n] = (int16_t)t;
@@ -177,7 +183,7 @@ __global__ __launch_bounds__(64 * GEMV_MAX_WAVES) void linear_gemv(LinearArgs p)
       e.rq_m = p.rq[2 * nn];
       e.rq_s = p.rq[2 * nn + 1];
       e.bias = p.bias ? p.bias[nn] : 0;
-      if (EPI == EPI_RESADD || EPI == EPI_MUL) {
+      if (EPI == EPI_RESADD || EPI == EPI_MUL || EPI == EPI_ADD) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int m = m0 + 4 * kg + r;
@@ -258,7 +264,7 @@ __global__ __launch_bounds__(64) void linear_gemv1(LinearArgs p) {
   const v2i rq = ld8(rsrc(p.rq, (int64_t)p.N * 8), lead ? 8 * n : LD_OOB);
   const int32_t bias = ld4(rsrc(p.bias, (int64_t)p.N * 4), lead ? 4 * n : LD_OOB);
   const int32_t aux =
-      (EPI == EPI_RESADD || EPI == EPI_MUL) ? ld2s(rsrc(p.aux, (int64_t)p.N * 2), lead ? 2 * n : LD_OOB) : 0;
+      (EPI == EPI_RESADD || EPI == EPI_MUL || EPI == EPI_ADD) ? ld2s(rsrc(p.aux, (int64_t)p.N * 2), lead ? 2 * n : LD_OOB) : 0;
   issue_fence();
   int32_t acc = 0;
 #pragma unroll
@@ -291,7 +297,10 @@ __global__ __launch_bounds__(64) void linear_gemv1(LinearArgs p) {
     return;
   }
   int64_t t = sat16(v);
-  if (EPI == EPI_RESADD) t = sat16(t + aux);
+  if (EPI == EPI_ADD) {
+    p.pre[n] = (int16_t)t;
+    t = sat16(rshr32_any((int32_t)t, p.aux_shift) + aux);
+  } else if (EPI == EPI_RESADD) t = sat16(t + aux);
   else if (EPI == EPI_SILU) t = silu16(t, p.Mi, p.Si, p.sh);
   else if (EPI == EPI_MUL) t = sat16(rshr(wmul(t, aux), p.aux_shift));
   static_cast<int16_t*>(p.out)[n] = (int16_t)t;
@@ -1589,10 +1598,17 @@ static int launch_mfma_shape(LinearArgs& p, void* ws, hipStream_t stream, const 
   return launch_mfma<EPI, OUT8, 64, 128, 4, KT>(p, ws, stream, norm, norm_done);
 }
 
+static bool rows_in_blocks16(const LinearArgs& p, bool aligned) {
+  return p.M <= 1024 && aligned && p.K <= 3072 && ceil_div(p.M, 16) * (int64_t)p.N * p.K <= (16ll << 20);
+}
+static bool linear_aligned(const LinearArgs& p) {
+  return p.K % 16 == 0 && p.lda % 16 == 0 && (uintptr_t)p.A % 16 == 0 && (uintptr_t)p.W % 16 == 0;
+}
+
 template <int EPI, bool OUT8>
 static int launch_linear(LinearArgs& p, void* ws, hipStream_t stream, const NormQuant* norm = nullptr,
                          bool* norm_done = nullptr) {
-  const bool aligned = (p.K % 16 == 0) && (p.lda % 16 == 0) && ((uintptr_t)p.A % 16 == 0) && ((uintptr_t)p.W % 16 == 0);
+  const bool aligned = linear_aligned(p);
   // More than 16 rows: the 16-row kernel over blocks of 16 rows (blockIdx.z) while re-reading W once
   // per block stays cheap -- every load of a workgroup is requested at entry, so it is one memory
   // round trip where an LDS ring is one per few K tiles.  Measured (us, 16-row blocks / MFMA tiles):
@@ -1601,22 +1617,23 @@ static int launch_linear(LinearArgs& p, void* ws, hipStream_t stream, const Norm
   // 7.0 / 6.1 (17 MB and more), 32 x 4864 x 896 9.7 / 8.7 (K past 3072: long serial chains per wave).
   // Rows that are normalised next (norm) keep the MFMA tiles where those split K (from K = 1024 on):
   // their finishing launch normalises too, which saves a launch.
-  const bool blocks16 = p.M > 16 && p.M <= 1024 && aligned && p.K <= 3072 && (!norm || p.K < 1024) &&
-                        ceil_div(p.M, 16) * (int64_t)p.N * p.K <= (16ll << 20);
-  if (p.M > 16 && p.K % 64 == 0 && aligned && !blocks16) {
-    if (p.K % 128 == 0) return launch_mfma_shape<EPI, OUT8, 128>(p, ws, stream, norm, norm_done);
-    return launch_mfma_shape<EPI, OUT8, 64>(p, ws, stream, norm, norm_done);
-  }
-  if (p.M > 16 && aligned && !blocks16) {
-    // 128x256 block tiles when they still fill the chip, else 128x128
-    const int mblocks = (int)ceil_div(p.M, 128);
-    const int nb256 = (int)ceil_div(p.N, 256), nb128 = (int)ceil_div(p.N, 128);
-    if ((int64_t)mblocks * nb256 >= 2 * current_cu_count())
-      hipLaunchKernelGGL((linear_tiled<EPI, OUT8, 2, 4>), dim3(mblocks * nb256), dim3(256), 0, stream, p, mblocks, nb256);
-    else
-      hipLaunchKernelGGL((linear_tiled<EPI, OUT8, 2, 2>), dim3(mblocks * nb128), dim3(256), 0, stream, p, mblocks, nb128);
-    LLHIP_LAUNCH_CHECK();
-    return 0;
+  const bool blocks16 = p.M > 16 && rows_in_blocks16(p, aligned) && (!norm || p.K < 1024);
+  if constexpr (EPI != EPI_ADD) {  // (llhip_linear_add comes here with rows of the kernels below only)
+    if (p.M > 16 && p.K % 64 == 0 && aligned && !blocks16) {
+      if (p.K % 128 == 0) return launch_mfma_shape<EPI, OUT8, 128>(p, ws, stream, norm, norm_done);
+      return launch_mfma_shape<EPI, OUT8, 64>(p, ws, stream, norm, norm_done);
+    }
+    if (p.M > 16 && aligned && !blocks16) {
+      // 128x256 block tiles when they still fill the chip, else 128x128
+      const int mblocks = (int)ceil_div(p.M, 128);
+      const int nb256 = (int)ceil_div(p.N, 256), nb128 = (int)ceil_div(p.N, 128);
+      if ((int64_t)mblocks * nb256 >= 2 * current_cu_count())
+        hipLaunchKernelGGL((linear_tiled<EPI, OUT8, 2, 4>), dim3(mblocks * nb256), dim3(256), 0, stream, p, mblocks, nb256);
+      else
+        hipLaunchKernelGGL((linear_tiled<EPI, OUT8, 2, 2>), dim3(mblocks * nb128), dim3(256), 0, stream, p, mblocks, nb128);
+      LLHIP_LAUNCH_CHECK();
+      return 0;
+    }
   }
   const int tiles = (int)ceil_div(p.N, 16);
   if (p.M == 1 && aligned && tiles < 2 * current_cu_count() && (int64_t)p.N * p.K < (1ll << 31)) {
@@ -1787,6 +1804,28 @@ extern "C" int llhip_linear(const int8_t* A, int64_t M, int64_t K, int64_t lda, 
     case EPI_MUL: return launch_linear<EPI_MUL, false>(p, ws, s);
     default: return launch_linear<EPI_NONE, false>(p, ws, s);
   }
+}
+
+extern "C" int llhip_linear_add(const int8_t* A, int64_t M, int64_t K, int64_t lda, const int8_t* W, int64_t N,
+                                const int32_t* rq, const int32_t* bias, const int16_t* a, int64_t sh_b, int16_t* o,
+                                int16_t* out, int64_t ld, void* ws, void* stream) {
+  if (!shift_ok(sh_b)) return fail(-EINVAL, "linear_add: shift out of [0,63]");
+  LinearArgs p{};
+  int rc = linear_args(p, A, M, K, lda, W, N, rq, bias, EPI_RESADD, a, ld, 0, 0, 0, 0, 0, out, ld);
+  if (rc) return rc < 0 ? rc : 0;
+  if (!o || ld != N) return fail(-EINVAL, "linear_add: contiguous rows of N values and the linear's own rows");
+  hipStream_t s = (hipStream_t)stream;
+  // one launch where the 16-row kernels run: their epilogue keeps both rows
+  const bool aligned = linear_aligned(p);
+  if (M <= 16 || rows_in_blocks16(p, aligned)) {
+    p.pre = o;
+    p.aux_shift = (int)sh_b;
+    return launch_linear<EPI_ADD, false>(p, ws, s);
+  }
+  p.aux = nullptr;
+  p.out = o;
+  rc = launch_linear<EPI_NONE, false>(p, ws, s);
+  return rc ? rc : llhip_vadd(a, o, M * N, sh_b, out, stream);
 }
 
 extern "C" int llhip_linear_norm(const int8_t* A, int64_t M, int64_t K, int64_t lda, const int8_t* W, int64_t N,

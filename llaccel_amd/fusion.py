@@ -117,6 +117,23 @@ class _RopeQuantStep:
                   self.model._stream_handle())
 
 
+class _LinearAddStep:
+    """An unfused graph's linear (epilogue none, i16 out) and the residual add of its output in one
+    llhip_linear_add call; both outputs are written."""
+
+    def __init__(self, model, lin, add, step):
+        self.model, self.lin, self.add = model, lin, add
+        self.kind, self.bytes_fn, self.name = step.kind, step.bytes_fn, step.name
+
+    def __call__(self, M, pos, pd=None):
+        m, o, a = self.model, self.lin, self.add
+        N, K = int(o["N"]), int(o["K"])
+        resid = a["a"] if a["b"] == o["out"] else a["b"]
+        _lib.call("llhip_linear_add", _vp(m._buf(o["in"])), M, K, K, _vp(m._dt[o["w"]]), N, _vp(m._dt[o["rq"]]),
+                  _vp(m._dt[o["bias"]]) if o.get("bias") else None, _vp(m._buf(resid)), int(a["sh_b"]),
+                  _vp(m._buf(o["out"])), _vp(m._buf(a["out"])), N, _vp(m._ws), m._stream_handle())
+
+
 class _LinearNormStep:
     """A resadd linear (i16 out) and the rmsnorm -> quant of its output rows in one
     llhip_linear_norm call (one finishing launch for both when the linear is split along K)."""
@@ -567,9 +584,28 @@ def fuse(model, ops, steps):
             out.append(st)
             src.append(None)
             i += n
+    _pair_linear_add(model, ops, out, src)
     _pair_linear_norm(model, ops, out, src)
     out.extend(steps[len(ops):])
     return out
+
+
+def _pair_linear_add(model, ops, out, src):
+    """A plain i16 linear followed by the add of its output to another activation (an unfused graph's o
+    and down projections) becomes one step: as the add's shifted operand b, or as a when sh_b = 0 (the
+    sum is then the same either way)."""
+    j = 0
+    while j + 1 < len(out):
+        i = src[j]
+        if i is not None and src[j + 1] == i + 1 and getattr(out[j], "kind", "") == "linear":
+            lin, add = ops[i], ops[i + 1]
+            if (_plain_linear(lin) and lin.get("out_dtype", "i16") == "i16" and getattr(out[j + 1], "kind", "") == "add"
+                    and add["a"] != add["b"] and add["out"] not in (lin["in"], lin["out"])
+                    and (add["b"] == lin["out"] or (add["a"] == lin["out"] and int(add["sh_b"]) == 0))):
+                out[j] = _LinearAddStep(model, lin, add, out[j])
+                src[j] = None
+                del out[j + 1], src[j + 1]
+        j += 1
 
 
 def _pair_linear_norm(model, ops, out, src):

@@ -287,6 +287,29 @@ def test_short_prompt_rows(M, K, N, epilogue, out_i8):
     assert np.array_equal(got, O.linear_c(a, w, rq, bias, out_i8, epilogue, aux, shift, silu))
 
 
+@pytest.mark.parametrize("sh_b", [0, 1, 5, 40])
+@pytest.mark.parametrize("M,K,N", [(1, 576, 576), (1, 64, 700), (3, 1536, 576), (16, 4864, 896), (1, 100, 33), (33, 592, 100),
+                                   (200, 896, 896), (200, 576, 4864)])
+def test_linear_add_equals_linear_then_vadd(M, K, N, sh_b):
+    """llhip_linear_add: the linear's own rows and the shifted sum, in one launch (16-row kernels, the
+    one-row kernel, unaligned K) and past their limits in two."""
+    from llaccel_amd import _lib
+    from tests.gpu_helpers import down, ptr, stream, torch, up, workspace
+
+    rng = np.random.default_rng(M + K + N + sh_b)
+    a, w, rq = _operands(rng, M, K, N, out_i8=False)
+    bias, res = rng.integers(-3000, 3000, N), rng.integers(-32768, 32768, (M, N))
+    ad, wd, rqd, bd, rd = up(a, np.int8), up(w, np.int8), up(rq, np.int32), up(bias, np.int32), up(res, np.int16)
+    o, x = (torch().zeros((M, N), dtype=torch().int16, device="cuda") for _ in range(2))
+    _lib.call("llhip_linear_add", ptr(ad), M, K, K, ptr(wd), N, ptr(rqd), ptr(bd), ptr(rd), sh_b, ptr(o), ptr(x), N,
+              ptr(workspace()), stream())
+    want = O.linear_c(a, w, rq, bias, False, "none", None, 0, None)
+    assert np.array_equal(down(o), want) and np.array_equal(down(x), O.vadd(res, want, sh_b))
+    with pytest.raises(ValueError):
+        _lib.call("llhip_linear_add", ptr(ad), M, K, K, ptr(wd), N, ptr(rqd), ptr(bd), ptr(rd), 64, ptr(o), ptr(x), N,
+                  ptr(workspace()), stream())
+
+
 @pytest.mark.parametrize("M,K,N", [(512, 4864, 896), (300, 2048, 576), (300, 896, 896), (40, 896, 896), (16, 896, 896),
                                    (16, 4864, 896), (5, 2048, 576), (2, 896, 1024), (512, 896, 896), (256, 1024, 576),
                                    (128, 896, 1024)])
