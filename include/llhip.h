@@ -112,6 +112,18 @@ typedef struct llhip_rope_quant_desc {
  * chunk's query rows, then its key rows with the layer's kv_write): the same checks and results as
  * the two calls in order. */
 int llhip_rope_quant2(const llhip_rope_quant_desc* a, const llhip_rope_quant_desc* b, void* stream);
+/* golden.py:287-293 + 141-158 + 119-120 [+ 344-351]  Q/K norm, then llhip_rope_quant2, in one launch: the
+ * heads of a->x (b->x) normalised as llhip_rmsnorm over M * H rows of D values (gamma i16 [D]), rotated,
+ * quantised and, for job b, written to the caches.  head_dim 64, 128 or 256; rows, tables, gammas and
+ * i16 outputs 16-byte, i8 rows and caches 8-byte aligned.  out (the normalised rows, i16 [M][H*D]) and
+ * the descriptors' y may be NULL: those rows are then not written. */
+typedef struct llhip_head_norm_desc {
+  const void* gamma;
+  int64_t eps_t, C, sh_post;
+  void* out;
+} llhip_head_norm_desc;
+int llhip_norm_rope_quant2(const llhip_rope_quant_desc* a, const llhip_head_norm_desc* na,
+                           const llhip_rope_quant_desc* b, const llhip_head_norm_desc* nb, void* stream);
 
 /* ---- gemm engine ---- */
 /* golden.py:316-342  out[M][N] = epilogue(requant(A[M][K] . W[N][K]^T + bias)).

@@ -62,6 +62,7 @@ _SIGS = {
     "llhip_rope_quant": [_p, _i64, _i64, _i64, _i64, _p, _p, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _p, _p, _i64, _p,
                          _i64, _i64, _p],
     "llhip_rope_quant2": [_p, _p, _p],
+    "llhip_norm_rope_quant2": [_p, _p, _p, _p, _p],
     "llhip_quant_rows_i8": [_p, _i64, _i64, _i64, _p, _i64, _p, _p, _p],
     "llhip_f32_absmax": [_p, _i64, _i64, _i64, _p, _p, _p, _p],
     "llhip_f32_rms_min": [_p, _i64, _i64, _p, _p],
@@ -150,6 +151,11 @@ class RopeQuantDesc(ctypes.Structure):
                 ("table_rows", _i64), ("pos", _i64), ("pos_dev", _p), ("row_pos", _p), ("y", _p), ("yq", _p),
                 ("qM", _i64), ("qS", _i64), ("kc", _p), ("v", _p), ("ldv", _i64), ("vc", _p), ("max_seq", _i64),
                 ("slot_stride", _i64), ("seq_rows", _i64)]
+
+
+class HeadNormDesc(ctypes.Structure):
+    """llhip_head_norm_desc: the Q or K norm of llhip_norm_rope_quant2."""
+    _fields_ = [("gamma", _p), ("eps_t", _i64), ("C", _i64), ("sh_post", _i64), ("out", _p)]
 
 
 class LinearProblem(ctypes.Structure):

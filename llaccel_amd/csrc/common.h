@@ -256,18 +256,42 @@ __device__ __forceinline__ int load_pos(const int32_t* pos_dev, int pos) {
 // compiler issues its argument loads lazily, between dependent steps, and each first touch of a
 // line would cost a memory round trip (every graph launch has its own argument buffer); after
 // this they hit the scalar cache.
+// The loads and their wait are one asm block: a block that only issued them would leave its output
+// registers to the compiler while the loads are still in flight.
 template <int BYTES>
 __device__ __forceinline__ void kernarg_warm() {
   static_assert(BYTES <= 768, "at most 12 argument lines");
+  constexpr int LINES = (BYTES + 63) / 64;
   auto kp = __builtin_amdgcn_kernarg_segment_ptr();
-  int d[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-  for (int i = 0; i < 12; ++i)
-    if (64 * i < BYTES) __asm__ volatile("s_load_dword %0, %1, %2" : "=s"(d[i]) : "s"(kp), "i"(64 * i));
-  // the loaded words are inputs of the wait so that they occupy distinct registers
-  __asm__ volatile("s_waitcnt lgkmcnt(0)" ::"s"(d[0]), "s"(d[1]), "s"(d[2]), "s"(d[3]), "s"(d[4]), "s"(d[5]), "s"(d[6]),
-                   "s"(d[7]), "s"(d[8]), "s"(d[9]), "s"(d[10]), "s"(d[11])
-                   : "memory");
+  int d;
+#define LLHIP_KW0
+#define LLHIP_KW1 LLHIP_KW0 "s_load_dword %0, %1, 0x0\n"
+#define LLHIP_KW2 LLHIP_KW1 "s_load_dword %0, %1, 0x40\n"
+#define LLHIP_KW3 LLHIP_KW2 "s_load_dword %0, %1, 0x80\n"
+#define LLHIP_KW4 LLHIP_KW3 "s_load_dword %0, %1, 0xc0\n"
+#define LLHIP_KW5 LLHIP_KW4 "s_load_dword %0, %1, 0x100\n"
+#define LLHIP_KW6 LLHIP_KW5 "s_load_dword %0, %1, 0x140\n"
+#define LLHIP_KW7 LLHIP_KW6 "s_load_dword %0, %1, 0x180\n"
+#define LLHIP_KW8 LLHIP_KW7 "s_load_dword %0, %1, 0x1c0\n"
+#define LLHIP_KW9 LLHIP_KW8 "s_load_dword %0, %1, 0x200\n"
+#define LLHIP_KW10 LLHIP_KW9 "s_load_dword %0, %1, 0x240\n"
+#define LLHIP_KW11 LLHIP_KW10 "s_load_dword %0, %1, 0x280\n"
+#define LLHIP_KW12 LLHIP_KW11 "s_load_dword %0, %1, 0x2c0\n"
+#define LLHIP_KW(n) \
+  if constexpr (LINES == n) __asm__ volatile(LLHIP_KW##n "s_waitcnt lgkmcnt(0)" : "=&s"(d) : "s"(kp) : "memory")
+  LLHIP_KW(1);
+  LLHIP_KW(2);
+  LLHIP_KW(3);
+  LLHIP_KW(4);
+  LLHIP_KW(5);
+  LLHIP_KW(6);
+  LLHIP_KW(7);
+  LLHIP_KW(8);
+  LLHIP_KW(9);
+  LLHIP_KW(10);
+  LLHIP_KW(11);
+  LLHIP_KW(12);
+#undef LLHIP_KW
 }
 // wave index as a scalar (uniform) value, so per-wave buffer descriptors stay in SGPRs
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }

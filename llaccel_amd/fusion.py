@@ -17,6 +17,7 @@ Recognised runs (the op order the reference's quantizer and compiler emit, refqu
 """
 from __future__ import annotations
 
+import collections
 import ctypes
 
 from . import _lib
@@ -72,11 +73,18 @@ class _NormQuantStep:
     def __init__(self, model, rn, qu):
         self.model, self.rn, self.qu = model, rn, qu
         self.desc = _lib.NormQuantDesc()
+        self.dead = _dead(model, rn["out"])
+
+    def fill(self):
+        m = self.model
+        _pre(m, self.desc, self.rn, self.qu)
+        self.desc.prequant = 0
+        if self.dead and getattr(m, "_lean", False):
+            self.desc.h_out = None
+        return self.desc
 
     def __call__(self, M, pos, pd=None):
-        _pre(self.model, self.desc, self.rn, self.qu)
-        self.desc.prequant = 0
-        _lib.call("llhip_rmsnorm_quant", ctypes.byref(self.desc), M, self.model._stream_handle())
+        _lib.call("llhip_rmsnorm_quant", ctypes.byref(self.fill()), M, self.model._stream_handle())
 
 
 class _RopeQuantStep:
@@ -117,6 +125,30 @@ class _RopeQuantStep:
                   self.model._stream_handle())
 
 
+class _HeadNormRopeStep:
+    """The Q/K norms, rope and quant of the q and k rows and the layer's kv_write (head_dim 64, 128 or 256)
+    in one llhip_norm_rope_quant2 launch."""
+
+    def __init__(self, model, norms, rope):
+        self.model, self.norms, self.rope = model, norms, rope
+        self.desc = (_lib.HeadNormDesc(), _lib.HeadNormDesc())
+        self.dead = [(_dead(model, n["out"]), _dead(model, ro["out"])) for n, (ro, _, _) in zip(norms, rope.parts)]
+
+    def __call__(self, M, pos, pd=None):
+        m, r = self.model, self.rope
+        lean = getattr(m, "_lean", False)
+        for d, n, rd, rn, (dead, rope_dead) in zip(r.desc, self.desc, r.parts, self.norms, self.dead):
+            r._fill(d, *rd, M, pos, pd)
+            d.x = _vp(m._buf(rn["in"]))
+            n.gamma = _vp(m._dt[rn["gamma"]])
+            n.eps_t, n.C, n.sh_post = int(rn["eps_t"]), int(rn["C"]), int(rn["sh_post"])
+            n.out = None if lean and dead else _vp(m._buf(rn["out"]))
+            if lean and rope_dead:
+                d.y = None
+        _lib.call("llhip_norm_rope_quant2", ctypes.byref(r.desc[0]), ctypes.byref(self.desc[0]), ctypes.byref(r.desc[1]),
+                  ctypes.byref(self.desc[1]), m._stream_handle())
+
+
 class _LinearAddStep:
     """An unfused graph's linear (epilogue none, i16 out) and the residual add of its output in one
     llhip_linear_add call; both outputs are written."""
@@ -144,8 +176,7 @@ class _LinearNormStep:
 
     def __call__(self, M, pos, pd=None):
         m, o = self.model, self.lin
-        _pre(m, self.norm.desc, self.norm.rn, self.norm.qu)
-        self.norm.desc.prequant = 0
+        self.norm.fill()
         N, K = int(o["N"]), int(o["K"])
         out, aux = m._buf(o["out"]), m._buf(o["aux"])
         _lib.call("llhip_linear_norm", _vp(m._buf(o["in"])), M, K, K, _vp(m._dt[o["w"]]), N, _vp(m._dt[o["rq"]]),
@@ -198,6 +229,7 @@ class _GroupRopeStep:
 
     def __init__(self, model, group, rope):
         self.model, self.group, self.rope = model, group, rope
+        self.dead = [_dead(model, ro["out"]) for ro, _, _ in rope.parts]
         self.fused = True   # cleared once the fused entry refuses this graph's operands
         self.launched = 0   # fused launches made (a test hook)
 
@@ -205,8 +237,10 @@ class _GroupRopeStep:
         if self.fused:
             g, r, m = self.group, self.rope, self.model
             g.fill()
-            for d, (ro, qu, kvw) in zip(r.desc, r.parts):
+            for d, (ro, qu, kvw), dead in zip(r.desc, r.parts, self.dead):
                 r._fill(d, ro, qu, kvw, M, pos, pd)
+                if dead and getattr(m, "_lean", False):
+                    d.y = None  # the rotated rows stay in registers (the linears' rows are written)
             a = g.lins[0]
             try:
                 _lib.call("llhip_linear_group_rope", _vp(m._buf(a["in"])), M, int(a["K"]), int(a["K"]), g.probs,
@@ -260,8 +294,18 @@ class _GateUpStep:
 
 
 def _reads(model, name: str) -> int:
-    """How many ops of the model's op list read activation `name`."""
-    return sum(1 for o in model.q.ops for k, v in o.items() if k not in ("op", "out") and isinstance(v, str) and v == name)
+    """How many ops of the model's op list read activation `name` (counted once per op list)."""
+    counts = getattr(model, "_read_counts", None)
+    if counts is None:
+        counts = model._read_counts = collections.Counter(
+            v for o in model.q.ops for k, v in o.items() if k not in ("op", "out") and isinstance(v, str))
+    return counts[name]
+
+
+def _dead(model, name: str) -> bool:
+    """Nothing but the op after it reads activation `name` (its fused launch keeps the value in
+    registers): a launch that collects no activations (model._lean) need not write it."""
+    return _reads(model, name) == 1 and name != model.q.output_name
 
 
 def _gate_up(model, ops, i):
@@ -279,11 +323,41 @@ def _gate_up(model, ops, i):
     return _GateUpStep(model, g, u, q)
 
 
+def _rope_group(model, rq_, rk_, qq_, kq_, kvw) -> bool:
+    """The five ops are rope q, rope k, quant q, quant k of their outputs and the kv_write of the keys."""
+    return (_is(rq_, "rope") and _is(rk_, "rope") and _is(qq_, "quant") and _is(kq_, "quant") and _is(kvw, "kv_write")
+            and qq_["in"] == rq_["out"] and kq_["in"] == rk_["out"] and kvw["k"] == kq_["out"]
+            and int(kvw["Hkv"]) == int(rk_["H"]) and int(kvw["D"]) == int(rk_["D"])
+            and model._act_spec[kvw["v"]][1] >= int(rk_["H"]) * int(rk_["D"]))
+
+
+def _head_norms(model, ops, i):
+    """ops[i:i+7] = the rmsnorms of the q and k heads, then a rope group over their outputs."""
+    if i + 6 >= len(ops):
+        return None
+    nq, nk, rq_, rk_, qq_, kq_, kvw = ops[i:i + 7]
+    if not (_is(nq, "rmsnorm") and _is(nk, "rmsnorm") and _rope_group(model, rq_, rk_, qq_, kq_, kvw)):
+        return None
+    D = int(rq_["D"])
+    if D not in (64, 128, 256) or int(rk_["D"]) != D or rq_["in"] != nq["out"] or rk_["in"] != nk["out"]:
+        return None
+    for n, r in ((nq, rq_), (nk, rk_)):
+        if int(n.get("heads", 1)) != int(r["H"]) or int(model._dt[n["gamma"]].shape[0]) != D:
+            return None
+    dt = model._dt  # views into the qgraph's blob at its offsets, which need not be aligned
+    if any(dt[t].data_ptr() % 16 for t in (nq["gamma"], nk["gamma"], "rope_cos", "rope_sin")):
+        return None
+    if model._act_spec[kvw["v"]][1] % 8:
+        return None
+    return _HeadNormRopeStep(model, (nq, nk), _RopeQuantStep(model, rq_, qq_, rk_, kq_, kvw))
+
+
 def wide_steps(model, ops, steps):
     """Launches of a fused run for more rows than its fused kernel takes (prompt chunks): the run's
     per-op steps, with each rmsnorm + quant as one launch, three linears of one input
     (q, k, v) as one grouped launch, the gate and up linears and the quant of their product as
-    one launch, and attn_in's group rope q, rope k, quant q, quant k, kv_write as one.  The
+    one launch, and attn_in's group rope q, rope k, quant q, quant k, kv_write as one (with the Q/K
+    norms before it where it has them).  The
     arithmetic of every op is unchanged."""
     out, i = [], 0
     while i < len(ops):
@@ -307,12 +381,14 @@ def wide_steps(model, ops, steps):
                 out.append(_GroupLinearStep(model, lins))
                 i += 3
                 continue
+        hn = _head_norms(model, ops, i)
+        if hn is not None:
+            out.append(hn)
+            i += 7
+            continue
         if i + 4 < len(ops):
             rq_, rk_, qq_, kq_, kvw = ops[i:i + 5]
-            if (_is(rq_, "rope") and _is(rk_, "rope") and _is(qq_, "quant") and _is(kq_, "quant")
-                    and _is(kvw, "kv_write") and qq_["in"] == rq_["out"] and kq_["in"] == rk_["out"]
-                    and kvw["k"] == kq_["out"] and int(kvw["Hkv"]) == int(rk_["H"]) and int(kvw["D"]) == int(rk_["D"])
-                    and model._act_spec[kvw["v"]][1] >= int(rk_["H"]) * int(rk_["D"])):
+            if _rope_group(model, rq_, rk_, qq_, kq_, kvw):
                 rope = _RopeQuantStep(model, rq_, qq_, rk_, kq_, kvw)
                 prev = out[-1] if out else None
                 if (isinstance(prev, _GroupLinearStep) and int(rq_["D"]) == 64
