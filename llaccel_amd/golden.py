@@ -966,44 +966,71 @@ class GoldenModel:
 
     PF_GRAPHS = 16  # whole-prompt prefill graphs kept (oldest dropped first)
 
-    def _prefill_launch(self, tokens, M: int) -> None:
-        """The whole-prompt prefill launch of `tokens` padded to M rows at positions 0..M-1.  Its
-        ~300 kernel launches are enqueued by the host in about as long as the GPU runs them, so
-        the second prefill of a (rows, prompt length, KV slot) shape captures them in a HIP graph
-        and every later one replays it, after copying the token ids into the graph's buffer."""
+    def _prefill_launch(self, tokens, M: int):
+        """The whole-prompt prefill launch of `tokens` padded to M rows at positions 0..M-1; returns the
+        M x vocab_padded logits rows in a buffer of their own.  Its ~200 kernel launches are enqueued
+        by the host in about as long as the GPU runs them, so the second prefill of a (rows, prompt
+        length, KV slot) shape captures them in a HIP graph and every later one replays it, after
+        copying the token ids into the graph's buffer.  The plan's last step, when it is the head's
+        (norm, lm_head), is launched outside the graph: the lm_head then writes each call's rows where
+        they stay, instead of into the graph's buffer that a copy would have to empty (512 x 151936
+        rows: 54 us of 1.64 ms; 1531 rows 167 us of 1.9 ms)."""
         self._lean = True  # no activation is collected here: dead intermediates go unwritten
         try:
-            self._prefill_launch_rows(tokens, M)
+            return self._prefill_launch_rows(tokens, M)
         finally:
             self._lean = False
 
-    def _prefill_launch_rows(self, tokens, M: int) -> None:
-        key = (M, len(tokens), self._slot)
-        if not self.use_graph:
-            self._launch_tokens(tokens, 0, M)
-            return
+    def _head_step(self, M: int):
+        """The plan's last step when it alone writes the logits, over rows a prompt has; else None."""
+        last = self._plan[-1] if self._plan else None
+        if getattr(last, "kind", "") == "norm_linear" and last.takes_wide(M) and last.name == self.q.output_name:
+            return last
+        return None
+
+    def _prefill_body(self, tokens, n: int, M: int, head) -> None:
+        """Embedding gather of n device tokens and the plan's steps, without the head's step."""
+        _lib.call("llhip_embed_rows", _ptr(self._dt["embed"]), self.embed.shape[0], self.dim, _ptr(tokens), n, M,
+                  _ptr(self._act[self.q.input_name]), _stream())
+        for step in self._plan if head is None else self._plan[:-1]:
+            step(M, 0, None)
+
+    def _prefill_launch_rows(self, tokens, M: int):
         torch = _t()
         idx = self._token_rows(tokens)
+        if M > self.max_seq:
+            raise ValueError(f"positions 0..{M - 1} exceed max_seq={self.max_seq}")
         self._ensure_capacity(M)
-        g = self._pf_graphs.get(key)
-        if g is None:
+        head = self._head_step(M)
+        key = (M, len(tokens), self._slot)
+        g = self._pf_graphs.get(key) if self.use_graph else None
+        if g is None and self.use_graph:
             self._pf_seen[key] = self._pf_seen.get(key, 0) + 1
-            if self._pf_seen[key] < 2:
-                self._launch_tokens(tokens, 0, M)
-                return
-            tok = torch.zeros(max(len(idx), 1), dtype=torch.int32, device=self.device)
-            graph = torch.cuda.CUDAGraph()
-            with capture_graph(graph):
-                _lib.call("llhip_embed_rows", _ptr(self._dt["embed"]), self.embed.shape[0], self.dim, _ptr(tok),
-                          len(idx), M, _ptr(self._act[self.q.input_name]), _stream())
-                self._execute(M, 0)
-            while len(self._pf_graphs) >= self.PF_GRAPHS:
-                self._pf_graphs.pop(next(iter(self._pf_graphs)))
-            g = self._pf_graphs[key] = (graph, tok)
-        graph, tok = g
-        if len(idx):
-            tok.copy_(torch.from_numpy(np.ascontiguousarray(idx, dtype=np.int32)), non_blocking=False)
-        graph.replay()
+            if self._pf_seen[key] >= 2:
+                tok = torch.zeros(max(len(idx), 1), dtype=torch.int32, device=self.device)
+                graph = torch.cuda.CUDAGraph()
+                with capture_graph(graph):
+                    self._prefill_body(tok, len(idx), M, head)
+                while len(self._pf_graphs) >= self.PF_GRAPHS:
+                    self._pf_graphs.pop(next(iter(self._pf_graphs)))
+                g = self._pf_graphs[key] = (graph, tok)
+        if g is None:
+            self._prefill_body(_up(idx if len(idx) else np.zeros(1, np.int32), np.int32), len(idx), M, head)
+        else:
+            graph, tok = g
+            if len(idx):
+                tok.copy_(torch.from_numpy(np.ascontiguousarray(idx, dtype=np.int32)), non_blocking=False)
+            graph.replay()
+        shared = self._act[self.q.output_name]
+        if head is None:
+            return shared[:M].clone()
+        rows = torch.empty((M, shared.shape[1]), dtype=shared.dtype, device=self.device)
+        self._act[self.q.output_name] = rows
+        try:
+            head(M, 0, None)
+        finally:
+            self._act[self.q.output_name] = shared
+        return rows
 
     # ---- device-resident greedy decode ----------------------------------------------------
     def _decode_state(self, ring_cap: int) -> None:
@@ -1319,9 +1346,8 @@ class GoldenModel:
         L = len(tokens)
         padded = -(-L // self.prefill_m) * self.prefill_m
         if acts is None and self.whole_prompt_prefill and L > self.prefill_m and padded <= self.max_seq:
-            self._prefill_launch(tokens, padded)
-            # a device copy of the L rows; each row crosses to the host when it is read
-            return DeviceRows(self._act[self.q.output_name][:L].clone())
+            # rows on the device; each crosses to the host when it is read
+            return DeviceRows(self._prefill_launch(tokens, padded)[:L])
         rows_out = []
         for start in range(0, len(tokens), self.prefill_m):
             chunk = tokens[start:start + self.prefill_m]
