@@ -338,6 +338,11 @@ typedef struct llhip_mlp_in_desc {
  * epilogue) [or linear g, linear u, silu, mul], quant. */
 int llhip_mlp_in(const llhip_mlp_in_desc* d, void* stream);
 
+#define LLHIP_BLOCK_ROWS_MAX 1024
+/* golden.py:286-309 + 332-342 -- llhip_mlp_in for up to LLHIP_BLOCK_ROWS_MAX rows (a short prompt), in
+ * blocks of 16 rows that each read the weights again. */
+int llhip_mlp_in_blocks(const llhip_mlp_in_desc* d, void* stream);
+
 typedef struct llhip_norm_linear_desc {
   llhip_norm_quant_desc pre;
   const void* W; const void* rq; const void* bias; const void* aux;

@@ -185,6 +185,7 @@ class NormLinearDesc(ctypes.Structure):
 
 
 _SIGS.update({
+    "llhip_mlp_in_blocks": [ctypes.POINTER(MlpInDesc), _p],
     "llhip_attn_in": [ctypes.POINTER(AttnInDesc), _p],
     "llhip_mlp_in": [ctypes.POINTER(MlpInDesc), _p],
     "llhip_norm_linear": [ctypes.POINTER(NormLinearDesc), _p],

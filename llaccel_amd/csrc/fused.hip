@@ -244,6 +244,13 @@ __device__ __forceinline__ void prerows_store(const NormQuant& pr, int M, const 
     *reinterpret_cast<v4i*>(a_lds + (c / nch) * lda + 16 * (c % nch)) = ld16(q, 16 * c);
 }
 
+// the rows from m0 on
+__device__ __forceinline__ void norm_rows_from(NormQuant& pr, int64_t m0) {
+  pr.x += m0 * pr.ldx;
+  if (pr.h_out) pr.h_out += m0 * pr.ldx;
+  if (pr.hq_out) pr.hq_out += m0 * pr.K;
+}
+
 // standalone rmsnorm + quant, one workgroup (256 threads) per row: thread t takes chunk t
 __global__ __launch_bounds__(256) void rmsnorm_quant_kernel(NormQuant pr) {
   __shared__ uint64_t part[4];
@@ -782,9 +789,21 @@ struct MlpInArgs {
 
 constexpr int WD_PF = 4;  // down-projection panel columns per thread loaded at kernel entry
 
-template <int MAXW>
+// BLK (more than 16 rows): workgroup (x, y) computes the rows 16 y .. 16 y + 15 alone, every row operand
+// and result moved on by 16 y rows.
+template <int MAXW, bool BLK = false>
 __global__ __launch_bounds__(64 * MAXW) void mlp_in_kernel(MlpInArgs p) {
   kernarg_warm<sizeof(MlpInArgs)>();
+  if constexpr (BLK) {
+    const int64_t m0 = 16 * (int64_t)blockIdx.y, o = m0 * p.N;
+    p.M = min(16, p.M - (int)m0);
+    norm_rows_from(p.pre, m0);
+    if (p.g_out) p.g_out += o;
+    if (p.u_out) p.u_out += o;
+    p.sg_out += o;
+    p.f_out += o;
+    p.fq_out += o;
+  }
   extern __shared__ __attribute__((aligned(16))) int8_t dyn[];
   __shared__ v4i red[MAXW][64];
   __shared__ uint32_t sig32[129];
@@ -1401,6 +1420,28 @@ extern "C" int llhip_mlp_in(const llhip_mlp_in_desc* d, void* stream) {
   }
   hipLaunchKernelGGL((mlp_in_kernel<FUSED_WAVES>), dim3((unsigned)ceil_div(p.N, 16)), dim3(128 * p.KS),
                      (size_t)(p.M * (p.K + 16)), (hipStream_t)stream, p);
+  LLHIP_LAUNCH_CHECK();
+  return 0;
+}
+
+extern "C" int llhip_mlp_in_blocks(const llhip_mlp_in_desc* d, void* stream) {
+  if (!d) return fail(-EINVAL, "mlp_in: null descriptor");
+  int rc = 0;
+  if (d->M < 1 || d->M > LLHIP_BLOCK_ROWS_MAX) return fail(-EINVAL, "mlp_in: 1 to %d rows", LLHIP_BLOCK_ROWS_MAX);
+  if (d->M * d->pre.ldx >= (1ll << 30)) return fail(-EINVAL, "mlp_in: rows above 2 GiB");
+  // the rows normalised once when there are more workgroups than CUs, as in llhip_mlp_in
+  llhip_mlp_in_desc dd = *d;
+  const int64_t blocks = ceil_div(d->M, 16);
+  const bool apart = !d->pre.prequant && d->pre.hq_out && ceil_div(d->N, 16) * blocks > current_cu_count();
+  if (apart) dd.pre.prequant = 1;
+  dd.M = std::min<int64_t>(d->M, 16);
+  MlpInArgs p{};
+  rc = mlp_in_args(&dd, p, 0);
+  if (rc) return rc;
+  p.M = (int)d->M;
+  if (apart && (rc = llhip_rmsnorm_quant(&d->pre, d->M, stream))) return rc;
+  hipLaunchKernelGGL((mlp_in_kernel<FUSED_WAVES, true>), dim3((unsigned)ceil_div(p.N, 16), (unsigned)blocks),
+                     dim3(128 * p.KS), (size_t)(dd.M * (p.K + 16)), (hipStream_t)stream, p);
   LLHIP_LAUNCH_CHECK();
   return 0;
 }

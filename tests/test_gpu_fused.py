@@ -185,7 +185,7 @@ def test_prefill_batch_other_lengths_run_separately(tmp_path_factory):
 
 
 @pytest.mark.parametrize("K,N", [(576, 1536), (896, 4880), (1024, 48), (16, 32)])
-@pytest.mark.parametrize("M", [2, 3, 4, 5, 7, 8, 9, 13, 16])
+@pytest.mark.parametrize("M", [2, 3, 4, 5, 7, 8, 9, 13, 16, 17, 33, 128])
 def test_rows_normalised_in_the_prologue(M, K, N):
     """llhip_mlp_in of several rows normalising them in every workgroup (several waves to a row, one
     wave to one, two or more rows; past 8 rows and one workgroup per CU a launch of its own) writes
@@ -214,7 +214,13 @@ def test_rows_normalised_in_the_prologue(M, K, N):
         d.silu_Mi, d.silu_Si, d.silu_sh, d.mul_sh, d.fq_M, d.fq_S, d.M, d.N = 1 << 30, 30, 16, 11, 1 << 30, 37, M, N
         if pre:
             _lib.call("llhip_rmsnorm_quant", ctypes.byref(n), M, stream())
-        _lib.call("llhip_mlp_in", ctypes.byref(d), stream())
+        if M <= 16 or not pre:
+            _lib.call("llhip_mlp_in" if M <= 16 else "llhip_mlp_in_blocks", ctypes.byref(d), stream())
+        else:
+            for m in range(0, M, 16):
+                n.x, n.h_out, n.hq_out, d.M = ptr(x[m:]), ptr(h[m:]), ptr(hq[m:]), min(16, M - m)
+                d.sg_out, d.f_out, d.fq_out = ptr(sg[m:]), ptr(f[m:]), ptr(fq[m:])
+                _lib.call("llhip_mlp_in", ctypes.byref(d), stream())
         outs.append([a.cpu().numpy() for a in (h, hq, sg, f, fq)])
     for a, b in zip(*outs):
         assert np.array_equal(a, b)
