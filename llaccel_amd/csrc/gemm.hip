@@ -88,24 +88,18 @@ __device__ __forceinline__ void finish(const LinearArgs& p, int m, int n, int64_
   static_cast<int16_t*>(p.out)[(int64_t)m * p.ldo + n] = (int16_t)t;
 }
 
-// 16 bytes of a K-contiguous row starting at k (zeros past K)
-template <bool ALIGNED>
-__device__ __forceinline__ v4i load16(const int8_t* row, int k, int K, bool valid) {
-  if (ALIGNED) {
-    if (valid && k < K) return *reinterpret_cast<const v4i*>(row + k);
-    return v4i{0, 0, 0, 0};
-  } else {
-    uint32_t w[4] = {0, 0, 0, 0};
-    if (valid) {
+// 16 bytes of a K-contiguous row of any alignment starting at k (zeros past K)
+__device__ __forceinline__ v4i load16_bytes(const int8_t* row, int k, int K, bool valid) {
+  uint32_t w[4] = {0, 0, 0, 0};
+  if (valid) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        int kk = k + i;
-        uint32_t b = kk < K ? (uint8_t)row[kk] : 0u;
-        w[i >> 2] |= b << (8 * (i & 3));
-      }
+    for (int i = 0; i < 16; ++i) {
+      int kk = k + i;
+      uint32_t b = kk < K ? (uint8_t)row[kk] : 0u;
+      w[i >> 2] |= b << (8 * (i & 3));
     }
-    return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
   }
+  return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
 }
 
 // ---------------------------------------------------------------------------------------
@@ -148,36 +142,53 @@ constexpr int GEMV_PF = 8;  // K steps of W and A in flight per wave
 
 template <int EPI, bool OUT8, bool ALIGNED>
 __global__ __launch_bounds__(64 * GEMV_MAX_WAVES) void linear_gemv(LinearArgs p) {
+  kernarg_warm<sizeof(LinearArgs)>();
   __shared__ v4i red[GEMV_MAX_WAVES - 1][64];
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = wave_id();
   const int nw = blockDim.x >> 6;
   const int col = lane & 15;
   const int kg = lane >> 4;
   const int tile = blockIdx.x;  // columns [tile * cpb, tile * cpb + cpb): lanes col >= cpb carry zero weights
   const int m0 = blockIdx.z * 16;
-  const int n = tile * p.cpb + col;
+  const int n0 = tile * p.cpb, n = n0 + col;
   const bool nvalid = col < p.cpb && n < p.N;
   const int nn = nvalid ? n : 0;
   const bool avalid = m0 + col < p.M;
   const int8_t* wrow = p.W + (int64_t)nn * p.K;
   const int8_t* arow = p.A + (int64_t)(avalid ? m0 + col : 0) * p.lda;
+  // ALIGNED: the tile's rows of W and A as buffers, so that a lane without a column, a row or a K
+  // step left reads zeros without a branch around its loads; a launch is one round trip of loads and
+  // what comes before them.  With the argument lines read at entry, against a branch per load: 3 rows
+  // of 576 and 1536 with the residual add 3.9 -> 3.2 us, 16 rows of 896 and 4864 5.5 -> 5.3, 64 rows
+  // of 576 4.0 -> 3.8
+  const int cols = min(p.cpb, p.N - n0), rows = min(16, p.M - m0);
+  const Rsrc wr = rsrc(p.W + (int64_t)n0 * p.K, (int64_t)cols * p.K);
+  const Rsrc ar = rsrc(p.A + (int64_t)m0 * p.lda, (rows - 1) * p.lda + p.K);
+  const uint32_t woff = (uint32_t)(col * p.K), aoff = (uint32_t)(col * (int)p.lda);
 
   const int spw = (p.steps + nw - 1) / nw;
   const int s_begin = min(wave * spw, p.steps);
   const int s_end = min(s_begin + spw, p.steps);
+  const int k_end = min(s_end * 64, p.K);
+  const int wk = nvalid ? k_end : 0, ak = avalid ? k_end : 0;
+  auto load = [&](int s, v4i& b, v4i& a) {
+    const int k = s * 64 + kg * 16;
+    if constexpr (ALIGNED) {
+      b = ld16(wr, k < wk ? woff + k : LD_OOB);
+      a = ld16(ar, k < ak ? aoff + k : LD_OOB);
+    } else {
+      b = s < s_end ? load16_bytes(wrow, k, p.K, nvalid) : v4i{0, 0, 0, 0};
+      a = s < s_end ? load16_bytes(arow, k, p.K, avalid) : v4i{0, 0, 0, 0};
+    }
+  };
   v4i acc = {0, 0, 0, 0};
   int s = s_begin;
   // first GEMV_PF steps: every load issued before the first MFMA
   {
     v4i b[GEMV_PF], a[GEMV_PF];
 #pragma unroll
-    for (int u = 0; u < GEMV_PF; ++u) {
-      const int k = (s + u) * 64 + kg * 16;
-      const bool ok = s + u < s_end;
-      b[u] = ok ? load16<ALIGNED>(wrow, k, p.K, nvalid) : v4i{0, 0, 0, 0};
-      a[u] = ok ? load16<ALIGNED>(arow, k, p.K, avalid) : v4i{0, 0, 0, 0};
-    }
+    for (int u = 0; u < GEMV_PF; ++u) load(s + u, b[u], a[u]);
     EpiOperands<EPI> e{};
     if (wave == 0) {
       e.rq_m = p.rq[2 * nn];
@@ -186,8 +197,8 @@ __global__ __launch_bounds__(64 * GEMV_MAX_WAVES) void linear_gemv(LinearArgs p)
       if (EPI == EPI_RESADD || EPI == EPI_MUL || EPI == EPI_ADD) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int m = m0 + 4 * kg + r;
-          e.aux[r] = m < p.M ? p.aux[(int64_t)m * p.ldaux + nn] : (int16_t)0;
+          const int m = min(m0 + 4 * kg + r, p.M - 1);  // a row past M: read, not used
+          e.aux[r] = p.aux[(int64_t)m * p.ldaux + nn];
         }
       }
     }
@@ -198,12 +209,7 @@ __global__ __launch_bounds__(64 * GEMV_MAX_WAVES) void linear_gemv(LinearArgs p)
     for (; s < s_end; s += U) {
       v4i bb[U], aa[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int k = (s + u) * 64 + kg * 16;
-        const bool ok = s + u < s_end;
-        bb[u] = ok ? load16<ALIGNED>(wrow, k, p.K, nvalid) : v4i{0, 0, 0, 0};
-        aa[u] = ok ? load16<ALIGNED>(arow, k, p.K, avalid) : v4i{0, 0, 0, 0};
-      }
+      for (int u = 0; u < U; ++u) load(s + u, bb[u], aa[u]);
 #pragma unroll
       for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(aa[u], bb[u], acc, 0, 0, 0);
     }
@@ -1667,7 +1673,7 @@ static int launch_linear(LinearArgs& p, void* ws, hipStream_t stream, const Norm
     nw = (int)std::min<int64_t>(GEMV_MAX_WAVES, ceil_div(p.steps, GEMV_PF));
   }
   dim3 grid((unsigned)ceil_div(p.N, p.cpb), 1, zblocks);
-  if (aligned)
+  if (aligned && 16 * p.lda < (1ll << 31))  // 16 rows of A within a buffer's range
     hipLaunchKernelGGL((linear_gemv<EPI, OUT8, true>), grid, dim3(64 * nw), 0, stream, p);
   else
     hipLaunchKernelGGL((linear_gemv<EPI, OUT8, false>), grid, dim3(64 * nw), 0, stream, p);

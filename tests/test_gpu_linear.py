@@ -72,6 +72,26 @@ def test_ragged_shapes(M, K, N):
     assert np.array_equal(got, O.linear_c(a, w, rq, bias, False, "none", None, 0, None))
 
 
+@pytest.mark.parametrize("M,K,N,lda", [(1, 80, 1100, 96), (3, 80, 37, 96), (16, 592, 100, 640), (33, 592, 100, 1024),
+                                       (16, 1536, 4200, 1552), (2, 16, 1, 32)])
+def test_padded_rows_of_a(M, K, N, lda):
+    """Rows of A further apart than K, K not a multiple of the 64-value steps: nothing past a row is taken in."""
+    from llaccel_amd import _lib
+    from tests.gpu_helpers import down, ptr, stream, torch, up, workspace
+
+    t = torch()
+    rng = np.random.default_rng(M + K + N)
+    a, w, rq = _operands(rng, M, K, N, out_i8=False)
+    bias = rng.integers(-5000, 5000, N)
+    rows = rng.integers(-127, 128, (M, lda)).astype(np.int8)
+    rows[:, :K] = a
+    ad, wd, rqd, bd = up(rows, np.int8), up(w, np.int8), up(rq, np.int32), up(bias, np.int32)
+    out = t.empty((M, N), dtype=t.int16, device="cuda")
+    _lib.call("llhip_linear", ptr(ad), M, K, lda, ptr(wd), N, ptr(rqd), ptr(bd), 0, None, N, 0, 0, 0, 0, 0, ptr(out), N,
+              ptr(workspace()), stream())
+    assert np.array_equal(down(out), O.linear_c(a, w, rq, bias, False, "none", None, 0, None))
+
+
 def test_split_k_matches_unsplit_and_self_cleans():
     """The split-K path (workspace) and the one-wave-per-tile path give identical results, and
     repeated calls stay exact (the workspace is left zeroed)."""
