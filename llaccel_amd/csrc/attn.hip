@@ -166,8 +166,6 @@ __device__ __forceinline__ void wo_slice(const AttnArgs& p, int h, int ds, const
   }
 }
 
-__device__ __forceinline__ int32_t sbyte(int w, int i) { return (int32_t)(int8_t)((uint32_t)w >> (8 * i)); }
-
 template <int D>
 __device__ __forceinline__ int32_t dot_row(const v4i* qv, const v4i* kv) {
   constexpr int DC = D / 16;
@@ -195,8 +193,22 @@ __device__ __forceinline__ int32_t row_fold(int32_t v) {
 // exp LUTs staged in LDS: kExpI (16 u16 = 8 dwords) then kExpF (256 u16 = 128 dwords)
 constexpr int LUT_DW = 136;
 
-__device__ __forceinline__ uint32_t lut_prob_lds(int64_t z, const uint16_t* ei, const uint16_t* ef) {
-  if (z >= 4096 || z < 0) return 0u;
+// Probability of a key x = mx - s >= 0 below the row maximum (golden.py:170-172):
+// z = rshr(x * Ms, Ss) = (x * Ms + 2^(Ss-1)) >> Ss for x >= 0 (x < 2^24, Ms < 2^32: one 32x32->64
+// multiply-add), p = 0 past the 4096-entry exponent range, else the rounded LUT product.
+struct ProbParams {
+  uint32_t Ms;
+  int Ss;
+  uint64_t zc;  // 2^(Ss-1), or 0 when Ss = 0
+};
+
+__device__ __forceinline__ ProbParams prob_params(const AttnArgs& p) {
+  return ProbParams{(uint32_t)p.Ms, p.Ss, p.Ss > 0 ? 1ull << (p.Ss - 1) : 0ull};
+}
+
+__device__ __forceinline__ uint32_t prob_lds(int32_t x, const ProbParams& q, const uint16_t* ei, const uint16_t* ef) {
+  const uint64_t z = ((uint64_t)(uint32_t)x * q.Ms + q.zc) >> q.Ss;
+  if (z >= 4096) return 0u;
   const uint32_t zi = (uint32_t)z;
   return ((uint32_t)ei[zi >> 8] * (uint32_t)ef[zi & 255] + 32768u) >> 16;
 }
@@ -352,8 +364,9 @@ __global__ __launch_bounds__(ATTN_THREADS) void attention_rowhead(AttnArgs p) {
   const uint16_t* ei = reinterpret_cast<const uint16_t*>(lut32);
   const uint16_t* ef = ei + 16;
   uint32_t lsum = 0;
+  const ProbParams pq = prob_params(p);
   for (int t = tid; t < T; t += ATTN_THREADS) {
-    const uint32_t pr = lut_prob_lds(mulshift((int64_t)mx - sc[t], p.Ms, p.Ss), ei, ef);
+    const uint32_t pr = prob_lds(mx - sc[t], pq, ei, ef);
     sc[t] = (int32_t)pr;
     lsum += pr;
   }
@@ -364,34 +377,31 @@ __global__ __launch_bounds__(ATTN_THREADS) void attention_rowhead(AttnArgs p) {
 #pragma unroll
   for (int w = 0; w < ATTN_WAVES; ++w) total += (uint32_t)redsum[w];
   const uint32_t inv = 0x80000000u / (total > 1u ? total : 1u);  // 2^31 / total (golden.py:174)
-  const int32_t cap = (1 << p.pb) - 1;
+  const uint32_t cap = (1u << p.pb) - 1u;
   const int shp = 31 - p.pb;
-  for (int t = tid; t < T; t += ATTN_THREADS) {
-    const int64_t pn = rshr((int64_t)sc[t] * (int64_t)inv, shp);
-    sc[t] = (int32_t)(pn < cap ? pn : cap);
-  }
+  const uint64_t pc = 1ull << (shp - 1);
+  for (int t = tid; t < T; t += ATTN_THREADS)
+    sc[t] = (int32_t)min((uint32_t)(((uint64_t)(uint32_t)sc[t] * inv + pc) >> shp), cap);
   __syncthreads();
 
   // o[d] = sum_t pn[t] * v[t][d]: thread (tg, dc) takes keys tg, tg+TG, ... (prefetched rows
-  // first, then four in flight)
+  // first, then four in flight), two keys at a time, passes past the context skipped.  A 32-bit
+  // product per key and dimension is quarter rate (3 rows of about 70 keys, 9 heads of 64: 6.5 -> 4.8 us a
+  // launch; 16 rows of about 600 keys 7.3 -> 7.1)
   int32_t acc[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] = 0;
 #pragma unroll
-  for (int u = 0; u < VPF; ++u) {
+  for (int u = 0; u < VPF; u += 2) {
+    if (u * TG >= T) break;
     const int t = tg + u * TG;
-    const int32_t pn = t < T ? sc[t] : 0;
+    const uint32_t pa = t < T ? sc[t] : 0, pb = t + TG < T ? sc[t + TG] : 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      acc[i] += pn * sbyte(vpre[u].x, i);
-      acc[4 + i] += pn * sbyte(vpre[u].y, i);
-      acc[8 + i] += pn * sbyte(vpre[u].z, i);
-      acc[12 + i] += pn * sbyte(vpre[u].w, i);
-    }
+    for (int c = 0; c < 4; ++c) pv_pair(acc + 4 * c, pa | (pb << 16), vpre[u][c], vpre[u + 1][c]);
   }
   for (int ta = tg + VPF * TG; ta < T; ta += 4 * TG) {
     v4i vv[4];
-    int32_t pn[4];
+    uint32_t pn[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int t = ta + u * TG;
@@ -399,15 +409,12 @@ __global__ __launch_bounds__(ATTN_THREADS) void attention_rowhead(AttnArgs p) {
       pn[u] = t < T ? sc[t] : 0;
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < 4; u += 2)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        acc[i] += pn[u] * sbyte(vv[u].x, i);
-        acc[4 + i] += pn[u] * sbyte(vv[u].y, i);
-        acc[8 + i] += pn[u] * sbyte(vv[u].z, i);
-        acc[12 + i] += pn[u] * sbyte(vv[u].w, i);
-      }
+      for (int c = 0; c < 4; ++c) pv_pair(acc + 4 * c, pn[u] | (pn[u + 1] << 16), vv[u][c], vv[u + 1][c]);
   }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] >>= 8;
   // the lanes of a 16-lane row with equal lane % VDC hold the same 16 columns: fold them with
   // row rotations, then the 4 rows x ATTN_WAVES partials in LDS
 #pragma unroll
@@ -472,22 +479,6 @@ __device__ __forceinline__ uint32_t pack4(int32_t a, int32_t b, int32_t c, int32
   const uint32_t lo = __builtin_amdgcn_perm((uint32_t)b, (uint32_t)a, 0x0c0c0400u);
   const uint32_t hi = __builtin_amdgcn_perm((uint32_t)d, (uint32_t)c, 0x04000c0cu);
   return lo | hi;
-}
-
-// Probability of a key x = mx - s >= 0 below the row maximum (golden.py:170-172):
-// z = rshr(x * Ms, Ss) = (x * Ms + 2^(Ss-1)) >> Ss for x >= 0 (x < 2^24, Ms < 2^32: one 32x32->64
-// multiply-add), p = 0 past the 4096-entry exponent range, else the rounded LUT product.
-struct ProbParams {
-  uint32_t Ms;
-  int Ss;
-  uint64_t zc;  // 2^(Ss-1), or 0 when Ss = 0
-};
-
-__device__ __forceinline__ uint32_t prob_lds(int32_t x, const ProbParams& q, const uint16_t* ei, const uint16_t* ef) {
-  const uint64_t z = ((uint64_t)(uint32_t)x * q.Ms + q.zc) >> q.Ss;
-  if (z >= 4096) return 0u;
-  const uint32_t zi = (uint32_t)z;
-  return ((uint32_t)ei[zi >> 8] * (uint32_t)ef[zi & 255] + 32768u) >> 16;
 }
 
 // The rounded LUT product of every exponent index (golden.py:170-172): entry z < 4096 is
@@ -1300,11 +1291,12 @@ __global__ __launch_bounds__(ARF_THREADS) void attention_row_fused(AttnArgs p, i
   const int32_t mx = bc;
   const uint16_t* ei = reinterpret_cast<const uint16_t*>(lut32);
   const uint16_t* ef = ei + 16;
+  const ProbParams pq = prob_params(p);
   uint32_t pr[NK];
   uint32_t lsum = 0;
 #pragma unroll
   for (int i = 0; i < NK; ++i) {
-    pr[i] = t0 + k0 + KP * i < t1 ? lut_prob_lds(mulshift((int64_t)mx - sreg[i], p.Ms, p.Ss), ei, ef) : 0u;
+    pr[i] = t0 + k0 + KP * i < t1 ? prob_lds(mx - sreg[i], pq, ei, ef) : 0u;
     if (kc == 0) lsum += pr[i];
   }
   lsum = (uint32_t)wave_sum_i32((int)lsum);  // T * 65535 < 2^31
@@ -1327,21 +1319,24 @@ __global__ __launch_bounds__(ARF_THREADS) void attention_row_fused(AttnArgs p, i
   if (!ok_s) return;
   const uint32_t total = (uint32_t)bc;
   const uint32_t inv = 0x80000000u / (total > 1u ? total : 1u);  // 2^31 / total (golden.py:174)
-  const int32_t cap = (1 << p.pb) - 1;
+  const uint32_t cap = (1u << p.pb) - 1u;
   const int shp = 31 - p.pb;
-  // this split's value sums: 16 dimensions (chunk kc) of this thread's keys, then over the key groups
+  const uint64_t pc = 1ull << (shp - 1);
+  // this split's value sums: 16 dimensions (chunk kc) of this thread's keys, two keys at a time (one by
+  // one with 32-bit products 14.9 us a launch at 4080 keys, 14.3 so), then over the key groups
   int32_t o[16];
 #pragma unroll
   for (int j = 0; j < 16; ++j) o[j] = 0;
+  static_assert(NK % 2 == 0, "keys in pairs");
 #pragma unroll
-  for (int i = 0; i < NK; ++i) {
-    const int64_t q = rshr((int64_t)pr[i] * (int64_t)inv, shp);
-    const int32_t pn = (int32_t)(q < cap ? q : cap);
+  for (int i = 0; i < NK; i += 2) {
+    const uint32_t pa = min((uint32_t)(((uint64_t)pr[i] * inv + pc) >> shp), cap);
+    const uint32_t pb = min((uint32_t)(((uint64_t)pr[i + 1] * inv + pc) >> shp), cap);
 #pragma unroll
-    for (int j = 0; j < 16; ++j) o[j] += pn * (int32_t)(int8_t)((uint32_t)vreg[i][j >> 2] >> (8 * (j & 3)));
+    for (int c = 0; c < 4; ++c) pv_pair(o + 4 * c, pa | (pb << 16), vreg[i][c], vreg[i + 1][c]);
   }
 #pragma unroll
-  for (int j = 0; j < 16; ++j) part[k0][16 * kc + j] = o[j];
+  for (int j = 0; j < 16; ++j) part[k0][16 * kc + j] = o[j] >> 8;
   __syncthreads();
   if (tid < D) {
     int32_t sum = 0;

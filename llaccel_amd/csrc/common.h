@@ -293,6 +293,20 @@ __device__ __forceinline__ void kernarg_warm() {
   LLHIP_KW(12);
 #undef LLHIP_KW
 }
+// o[j] += 256 (pa va[j] + pb vb[j]) over the four signed bytes of va and vb, with pn2 = pa | pb << 16 and
+// pa, pb < 2^15: the bytes go into the high halves of 16-bit pairs, so a pair costs one byte pick and
+// one full-rate v_dot2_i32_i16 where the 32-bit product of one key is a sign extension, a
+// quarter-rate multiply and an add.  Weighted sums of values by attention probabilities stay
+// below 2^31 in the scaled form: the probabilities of n keys add up to at most 2^15 + n / 2, so
+// |o| <= 2^30 + n 2^14, below 2^31 for n < 65536 keys of one thread.  The caller shifts the sum right by 8 (exact).
+__device__ __forceinline__ void pv_pair(int32_t* o, uint32_t pn2, int va, int vb) {
+  typedef short s2 __attribute__((ext_vector_type(2)));
+  const s2 p = __builtin_bit_cast(s2, pn2);
+#pragma unroll
+  for (uint32_t j = 0; j < 4; ++j)
+    o[j] = __builtin_amdgcn_sdot2(
+        p, __builtin_bit_cast(s2, __builtin_amdgcn_perm((uint32_t)vb, (uint32_t)va, 0x040C000Cu + 0x01000100u * j)), o[j], false);
+}
 // wave index as a scalar (uniform) value, so per-wave buffer descriptors stay in SGPRs
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 

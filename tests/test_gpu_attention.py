@@ -75,6 +75,23 @@ def test_attention_matches_oracle(M, H, Hkv, D, pos, max_seq):
     assert np.abs(got).max() > 0
 
 
+@pytest.mark.parametrize("D,H,Hkv", [(16, 4, 2), (64, 14, 2), (128, 16, 8), (256, 8, 2)])
+def test_one_row_context_edges(D, H, Hkv):
+    """One row, whose threads take its values two keys at a time: contexts of one key, and on both sides of a
+    whole pair, of the prefetched keys and of the loop past them; one-hot and flat probabilities."""
+    rng = np.random.default_rng(D)
+    max_seq = 1300
+    kc, vc = (rng.integers(-128, 128, (Hkv, max_seq, D)).astype(np.int8) for _ in range(2))
+    vc[:, ::3] = np.where(vc[:, ::3] < 0, -128, 127)
+    q = rng.integers(-128, 128, (1, H * D))
+    tg = 512 * 16 // D  # keys of one pass of the workgroup
+    for T in sorted({1, 2, 3, tg - 1, tg, tg + 1, 2 * tg + 1, 8 * tg, 8 * tg + 1, 9 * tg + 5, 1299} & set(range(1, max_seq))):
+        for Ss in (20, 31 + int(round(np.log2(5372 * np.sqrt(D) / 768))), 50):
+            got = gpu_attention(q, kc, vc, T - 1, H, Hkv, D, (1 << 31) - 1, Ss, 1 << 30, 38, 15)
+            want = O.attention_c(q, kc, vc, T - 1, H, Hkv, D, (1 << 31) - 1, Ss, 1 << 30, 38, 15)
+            assert np.array_equal(got, want), (T, Ss)
+
+
 def test_kv_write_and_positions():
     rng = np.random.default_rng(3)
     t = __import__("torch")
