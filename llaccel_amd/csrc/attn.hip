@@ -267,7 +267,10 @@ __global__ __launch_bounds__(ATTN_THREADS) void attention_rowhead(AttnArgs p) {
   // Loads in order of use: q and the keys of the first score pass, the LUT dwords (wave 0), the
   // value rows of this thread's first VPF keys.  The cache rows are addressed over the whole cache,
   // so these loads do not wait for the device position; rows at or past T are masked out below
-  // (their scores are never kept, their probabilities are zero).
+  // (their scores are never kept, their probabilities are zero).  Several rows (BOUND), whose
+  // workgroups fill the chip, wait for it once their first two key loads are on the way, and skip
+  // the loads past T: a workgroup of a short context otherwise reads 128 KB of stale cache (3 rows
+  // of about 70 keys 4.9 -> 4.4 us a launch, 16 rows of about 600 keys 7.4 -> 6.8).
   const int64_t slot = p.row_pos ? m * p.slot_stride : 0;
   const int8_t* kbase = p.kc + slot + (int64_t)g * p.max_seq * D;
   const int8_t* vbase = p.vc + slot + (int64_t)g * p.max_seq * D;
@@ -279,10 +282,27 @@ __global__ __launch_bounds__(ATTN_THREADS) void attention_rowhead(AttnArgs p) {
   constexpr int KPB = (64 / DC) * ATTN_WAVES;              // keys per block-wide load
   constexpr int KPF = (D <= 128 ? 1024 : 512) / KPB;      // loads per lane issued at entry
   const int kc = lane % DC, kw = wave * (64 / DC) + lane / DC;
+  constexpr bool BOUND = !WO;
+  // row m's context T = position + 1 (row m of a launch at pos sits at pos + m; with per-row
+  // positions, row m is its own sequence in cache slot m), never past the cache
+  auto context = [&] {
+    return min((p.row_pos ? *(const __attribute__((address_space(4))) int32_t*)(p.row_pos + m)
+                          : load_pos(p.pos_dev, p.pos) + m) + 1,
+               (int)p.max_seq);
+  };
+  int T = 0;
   const v4i qc = ld16(qr, 16 * kc);
   v4i kpf[KPF];
 #pragma unroll
-  for (int i = 0; i < KPF; ++i) kpf[i] = ld16(kr, (uint32_t)((i * KPB + kw) * D + 16 * kc));
+  for (int i = 0; i < KPF; i += 2) {
+    if (BOUND && i == (KPF > 2 ? 2 : 0)) T = context();
+    if (BOUND && i >= 2 && i * KPB >= T) {
+      kpf[i] = kpf[i + 1] = v4i{0, 0, 0, 0};
+      continue;
+    }
+    kpf[i] = ld16(kr, (uint32_t)((i * KPB + kw) * D + 16 * kc));
+    kpf[i + 1] = ld16(kr, (uint32_t)(((i + 1) * KPB + kw) * D + 16 * kc));
+  }
   issue_fence();
   uint32_t lw[3] = {0u, 0u, 0u};
   if (wave == 0) {  // (a load instruction costs address-unit cycles even when it reads nothing)
@@ -300,20 +320,25 @@ __global__ __launch_bounds__(ATTN_THREADS) void attention_rowhead(AttnArgs p) {
   const int dc = SLICE ? ds : tid % DC, tg = tid / VDC;
   v4i vpre[VPF];
 #pragma unroll
-  for (int u = 0; u < VPF; ++u) vpre[u] = ld16(vr, (uint32_t)((tg + u * TG) * D + 16 * dc));
+  for (int u = 0; u < VPF; u += 2) {
+    if (BOUND && u * TG >= T) {
+      vpre[u] = vpre[u + 1] = v4i{0, 0, 0, 0};
+      continue;
+    }
+    vpre[u] = ld16(vr, (uint32_t)((tg + u * TG) * D + 16 * dc));
+    vpre[u + 1] = ld16(vr, (uint32_t)((tg + (u + 1) * TG) * D + 16 * dc));
+  }
   issue_fence();
-  // row m's context T = position + 1 (row m of a launch at pos sits at pos + m; with per-row
-  // positions, row m is its own sequence in cache slot m), never past the cache.  A scalar load
-  // issued after the vector loads: a wait for it waits for every earlier scalar load.
-  const int T = min((p.row_pos ? *(const __attribute__((address_space(4))) int32_t*)(p.row_pos + m)
-                               : load_pos(p.pos_dev, p.pos) + m) + 1,
-                    (int)p.max_seq);
+  // One row: a scalar load issued after the vector loads (a wait for it waits for every earlier
+  // scalar load).
+  if (!BOUND) T = context();
   if (WO && h == 0 && m == 0 && ds == 0) zero_words(p.zero, p.zero_n);
 
   // scores s[t] = q . k[t] (int32, |s| <= D * 2^14)
   int32_t lmax = INT32_MIN;
 #pragma unroll
   for (int i = 0; i < KPF; ++i) {
+    if (BOUND && i * KPB >= T) break;
     const int t = i * KPB + kw;
     const int32_t sv = chunk_sum<DC>(dot16(qc, kpf[i]));
     if (kc == 0 && t < T) {
