@@ -160,8 +160,8 @@ __global__ __launch_bounds__(64 * GEMV_MAX_WAVES) void linear_gemv(LinearArgs p)
   // ALIGNED: the tile's rows of W and A as buffers, so that a lane without a column, a row or a K
   // step left reads zeros without a branch around its loads; a launch is one round trip of loads and
   // what comes before them.  With the argument lines read at entry, against a branch per load: 3 rows
-  // of 576 and 1536 with the residual add 3.9 -> 3.2 us, 16 rows of 896 and 4864 5.5 -> 5.3, 64 rows
-  // of 576 4.0 -> 3.8
+  // of 576 and 1536 with the residual add 3.9 -> 3.2 us, 64 rows of 576 4.0 -> 3.8 (16 rows of 896 and
+  // 4864 5.3 to 5.5 us both ways, by the box)
   const int cols = min(p.cpb, p.N - n0), rows = min(16, p.M - m0);
   const Rsrc wr = rsrc(p.W + (int64_t)n0 * p.K, (int64_t)cols * p.K);
   const Rsrc ar = rsrc(p.A + (int64_t)m0 * p.lda, (rows - 1) * p.lda + p.K);
