@@ -95,6 +95,7 @@ def test_oracle_errors_equal_reference_simulator(cid, img, pos, fusion, msg):
             dev.run(0, pos)
 
 
+@needs_ref
 @pytest.mark.parametrize("cid,img,pos,fusion,msg,sram_exact", C.partial_error_cases(),
                          ids=[c[0] for c in C.partial_error_cases()])
 def test_oracle_state_after_error_equals_reference_simulator(cid, img, pos, fusion, msg, sram_exact):
