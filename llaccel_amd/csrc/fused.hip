@@ -33,64 +33,35 @@ namespace llhip {
 // RMSNorm + quant prologue (golden.py:124-137, 119-120)
 // ---------------------------------------------------------------------------------------
 
-// Rows and 4-element output units of this wave.  With 2 M <= nw several waves share a row: each
-// computes the row's sum of squares (the row is 2 KiB at most) and applies the scale to its own
-// units, so no cross-wave reduction is needed.  Otherwise (full) wave w takes the rows w, w + nw, ...
-// whole, two at a time.
+// How a workgroup of nw waves gets its M quantised rows, one kernel instance each.  A kernel that held the
+// three forms had the registers of the largest: attn_in 129 VGPRs (three waves per SIMD) where one row
+// needs 78 and quantised rows 97, the head 127 with spills to scratch where they need 76 and 95 (896 x
+// 151936, one row 25.5 -> 23.9 us, 16 quantised rows 27.9 -> 26.5):
+//   NORM_SHARED  2 M <= nw: several waves share a row; each computes the row's sum of squares (the row
+//                is 2 KiB at most) and applies the scale to its own units, so no cross-wave reduction;
+//   NORM_ROWS    wave w takes the rows w, w + nw, ... whole, two at a time;
+//   NORM_QUANT   the rows come quantised from llhip_rmsnorm_quant.
+enum NormForm : int { NORM_SHARED = 0, NORM_ROWS = 1, NORM_QUANT = 2 };
+
+// Rows and 4-element output units of this wave (NORM_SHARED)
 struct NormMap {
-  int m0, step, j, G;  // rows m0, m0 + step, ...; units j*64 + lane + i*G*64
-  bool full;
+  int m0, j, G;  // row m0; units j*64 + lane + i*G*64
 };
 
 __device__ __forceinline__ NormMap norm_map(int M) {
   const int wave = wave_id(), nw = blockDim.x >> 6;
   NormMap r;
-  r.full = 2 * M > nw;
-  if (!r.full) {
-    r.m0 = wave % M;
-    r.step = M;
-    r.j = wave / M;
-    r.G = (nw - r.m0 + M - 1) / M;
-  } else {
-    r.m0 = wave;
-    r.step = nw;
-    r.j = 0;
-    r.G = 1;
-  }
+  r.m0 = wave % M;
+  r.j = wave / M;
+  r.G = (nw - r.m0 + M - 1) / M;
   return r;
 }
-
-// operands of the wave's first row (full: first two rows), loaded at kernel entry
-struct NormRegs {
-  v4i xs[2];   // 8-element chunks lane and lane + 64 (sum of squares; full: the whole row)
-  v2i xu, gu;  // x and gamma of the first output unit
-  v4i x1[2];   // full: the second row's chunks
-  v4i g[2];    // full: gamma chunks
-};
 
 // the 8-element chunks lane and lane + 64 of the row at byte offset `row`
 __device__ __forceinline__ void norm_row_load(Rsrc xr, uint32_t row, int nch, v4i (&x)[2]) {
   const int lane = threadIdx.x & 63;
   x[0] = ld16(xr, lane < nch ? row + 16 * lane : LD_OOB);
   x[1] = ld16(xr, lane + 64 < nch ? row + 16 * (lane + 64) : LD_OOB);
-}
-
-__device__ __forceinline__ void norm_prefetch(const NormQuant& pr, int M, const NormMap& nm, NormRegs& r) {
-  const int lane = threadIdx.x & 63, nch = pr.K >> 3, nu = pr.K >> 2;
-  const Rsrc xr = rsrc(pr.x, (int64_t)M * pr.ldx * 2), gr = rsrc(pr.gamma, (int64_t)pr.K * 2);
-  const uint32_t row = (uint32_t)(nm.m0 * pr.ldx * 2);
-  if (nm.full) {
-    if (nm.m0 >= M) return;  // this wave has no row
-    norm_row_load(xr, row, nch, r.xs);
-    if (nm.m0 + nm.step < M) norm_row_load(xr, row + (uint32_t)(nm.step * pr.ldx * 2), nch, r.x1);
-    norm_row_load(gr, 0, nch, r.g);
-    return;
-  }
-  r.xs[0] = ld16(xr, lane < nch ? row + 16 * lane : LD_OOB);
-  r.xs[1] = ld16(xr, lane + 64 < nch ? row + 16 * (lane + 64) : LD_OOB);
-  const int u = nm.j * 64 + lane;
-  r.xu = ld8(xr, u < nu ? row + 8 * u : LD_OOB);
-  r.gu = ld8(gr, u < nu ? 8 * u : LD_OOB);
 }
 
 __device__ __forceinline__ uint32_t norm_row_inv(const NormQuant& pr, const v4i& xs0, const v4i& xs1) {
@@ -159,90 +130,115 @@ __device__ __forceinline__ void norm_apply_row(const NormQuant& pr, int m, uint3
   }
 }
 
-// Rows m0, m0 + step, ... of this wave, two at a time so that the two rows' serial chains (sum,
-// square root, division) overlap; the first two from the registers loaded at entry, so that nothing
-// but the weights is waited for behind them.  Replaces a launch of its own for M > 1: a decode step
-// of 8 rows, 30 layers of 576, 894 -> 803 us; of 16 rows, 24 layers of 896: attn_in 7.0 + 2.9 us in two
-// launches, 8.8 us in one.
-__device__ __forceinline__ void norm_rows_full(const NormQuant& pr, const NormRegs& r, int M, const NormMap& nm,
-                                               int8_t* a_lds, int lda, bool write_global) {
-  const int nch = pr.K >> 3;
-  const Rsrc xr = rsrc(pr.x, (int64_t)M * pr.ldx * 2);
-  auto rows = [&](int m, const v4i (&x0)[2], const v4i (&x1)[2]) {
-    if (m + nm.step < M) {
-      const uint32_t i0 = norm_row_inv(pr, x0[0], x0[1]), i1 = norm_row_inv(pr, x1[0], x1[1]);
-      norm_apply_row(pr, m, i0, x0, r.g, a_lds, lda, write_global);
-      norm_apply_row(pr, m + nm.step, i1, x1, r.g, a_lds, lda, write_global);
-    } else {
-      norm_apply_row(pr, m, norm_row_inv(pr, x0[0], x0[1]), x0, r.g, a_lds, lda, write_global);
-    }
-  };
-  if (nm.m0 >= M) return;
-  rows(nm.m0, r.xs, r.x1);
-  for (int m = nm.m0 + 2 * nm.step; m < M; m += 2 * nm.step) {
-    v4i a[2], b[2];
-    norm_row_load(xr, (uint32_t)(m * pr.ldx * 2), nch, a);
-    norm_row_load(xr, (uint32_t)((m + nm.step) * pr.ldx * 2), nch, b);  // past row M - 1: zeros
-    rows(m, a, b);
-  }
-}
+// The rows' prologue in one of its forms: load() at kernel entry, store() leaves the quantised rows in
+// a_lds (the caller's barrier follows) and, from the workgroup that writes them, in h_out and hq_out.
+template <int FORM>
+struct NormStage;
 
-// The wave's first row and first unit use the registers loaded at entry in straight-line code,
-// so their waits cover those loads only; further units (K > 256 * waves sharing a row) load inside
-// loops.
-__device__ __forceinline__ void norm_quant_rows(const NormQuant& pr, const NormRegs& r, int M, const NormMap& nm,
-                                                int8_t* a_lds, int lda, bool write_global) {
-  if (nm.full) {
-    norm_rows_full(pr, r, M, nm, a_lds, lda, write_global);
-    return;
+// The row and first unit use the registers loaded at entry in straight-line code, so their waits
+// cover those loads only; further units (K > 256 * waves sharing a row) load inside loops.
+template <>
+struct NormStage<NORM_SHARED> {
+  NormMap nm;
+  v4i xs[2];   // the row's 8-element chunks lane and lane + 64 (sum of squares)
+  v2i xu, gu;  // x and gamma of the first output unit
+
+  __device__ __forceinline__ void load(const NormQuant& pr, int M) {
+    nm = norm_map(M);
+    const int lane = threadIdx.x & 63, nch = pr.K >> 3, nu = pr.K >> 2;
+    const Rsrc xr = rsrc(pr.x, (int64_t)M * pr.ldx * 2), gr = rsrc(pr.gamma, (int64_t)pr.K * 2);
+    const uint32_t row = (uint32_t)(nm.m0 * pr.ldx * 2);
+    norm_row_load(xr, row, nch, xs);
+    const int u = nm.j * 64 + lane;
+    xu = ld8(xr, u < nu ? row + 8 * u : LD_OOB);
+    gu = ld8(gr, u < nu ? 8 * u : LD_OOB);
   }
-  const int lane = threadIdx.x & 63, nu = pr.K >> 2;
-  const Rsrc xr = rsrc(pr.x, (int64_t)M * pr.ldx * 2), gr = rsrc(pr.gamma, (int64_t)pr.K * 2);
-  const int ustep = nm.G * 64;
-  {
-    const int m = nm.m0;
+
+  __device__ __forceinline__ void store(const NormQuant& pr, int M, int8_t* a_lds, int lda, bool write_global) {
+    const int lane = threadIdx.x & 63, nu = pr.K >> 2;
+    const Rsrc xr = rsrc(pr.x, (int64_t)M * pr.ldx * 2), gr = rsrc(pr.gamma, (int64_t)pr.K * 2);
+    const int m = nm.m0, ustep = nm.G * 64;
     const uint32_t row = (uint32_t)(m * pr.ldx * 2);
-    const uint32_t inv = norm_row_inv(pr, r.xs[0], r.xs[1]);
-    norm_apply_unit(pr, m, nm.j * 64 + lane, inv, r.xu, r.gu, a_lds, lda, write_global);
+    const uint32_t inv = norm_row_inv(pr, xs[0], xs[1]);
+    norm_apply_unit(pr, m, nm.j * 64 + lane, inv, xu, gu, a_lds, lda, write_global);
     for (int u0 = nm.j * 64 + ustep; u0 < nu; u0 += ustep) {
       const int u = u0 + lane;
-      const v2i xu = ld8(xr, u < nu ? row + 8 * u : LD_OOB), gu = ld8(gr, u < nu ? 8 * u : LD_OOB);
-      norm_apply_unit(pr, m, u, inv, xu, gu, a_lds, lda, write_global);
+      const v2i x = ld8(xr, u < nu ? row + 8 * u : LD_OOB), g = ld8(gr, u < nu ? 8 * u : LD_OOB);
+      norm_apply_unit(pr, m, u, inv, x, g, a_lds, lda, write_global);
     }
   }
-}
-
-// Rows already quantised by llhip_rmsnorm_quant (multi-row launches): the i8 rows [M][K] are
-// loaded at kernel entry (16-byte chunks, PRE_CHUNKS per thread) and staged in LDS.
-// Normalising M > 1 rows in every workgroup would repeat the whole row prologue per workgroup.
-constexpr int PRE_CHUNKS = 8;
-
-struct PreRows {
-  v4i c[PRE_CHUNKS];
 };
 
-__device__ __forceinline__ void prerows_load(const NormQuant& pr, int M, PreRows& r) {
-  const int nt = blockDim.x, tid = threadIdx.x, total = M * (pr.K >> 4);
-  const Rsrc q = rsrc(pr.hq_out, (int64_t)M * pr.K);
-#pragma unroll
-  for (int i = 0; i < PRE_CHUNKS; ++i) {
-    const int c = tid + i * nt;
-    r.c[i] = ld16(q, c < total ? 16 * c : LD_OOB);
-  }
-}
+// Two rows at a time so that their serial chains (sum, square root, division) overlap; the first two
+// from the registers loaded at entry, so that nothing but the weights is waited for behind them.
+// Replaces a launch of its own for M > 1: a decode step of 8 rows, 30 layers of 576, 894 -> 803 us.
+template <>
+struct NormStage<NORM_ROWS> {
+  v4i x0[2], x1[2];  // the wave's first two rows
+  v4i g[2];          // gamma
 
-__device__ __forceinline__ void prerows_store(const NormQuant& pr, int M, const PreRows& r, int8_t* a_lds, int lda) {
-  const int nt = blockDim.x, tid = threadIdx.x, nch = pr.K >> 4, total = M * nch;
-#pragma unroll
-  for (int i = 0; i < PRE_CHUNKS; ++i) {
-    const int c = tid + i * nt;
-    if (c < total) *reinterpret_cast<v4i*>(a_lds + (c / nch) * lda + 16 * (c % nch)) = r.c[i];
+  __device__ __forceinline__ void load(const NormQuant& pr, int M) {
+    const int m0 = wave_id(), nw = blockDim.x >> 6, nch = pr.K >> 3;
+    if (m0 >= M) return;  // this wave has no row
+    const Rsrc xr = rsrc(pr.x, (int64_t)M * pr.ldx * 2);
+    norm_row_load(xr, (uint32_t)(m0 * pr.ldx * 2), nch, x0);
+    if (m0 + nw < M) norm_row_load(xr, (uint32_t)((m0 + nw) * pr.ldx * 2), nch, x1);
+    norm_row_load(rsrc(pr.gamma, (int64_t)pr.K * 2), 0, nch, g);
   }
-  // small workgroups: the chunks beyond the prefetched ones
-  const Rsrc q = rsrc(pr.hq_out, (int64_t)M * pr.K);
-  for (int c = tid + PRE_CHUNKS * nt; c < total; c += nt)
-    *reinterpret_cast<v4i*>(a_lds + (c / nch) * lda + 16 * (c % nch)) = ld16(q, 16 * c);
-}
+
+  __device__ __forceinline__ void store(const NormQuant& pr, int M, int8_t* a_lds, int lda, bool write_global) {
+    const int m0 = wave_id(), nw = blockDim.x >> 6, nch = pr.K >> 3;
+    const Rsrc xr = rsrc(pr.x, (int64_t)M * pr.ldx * 2);
+    auto rows = [&](int m, const v4i (&a)[2], const v4i (&b)[2]) {
+      if (m + nw < M) {
+        const uint32_t i0 = norm_row_inv(pr, a[0], a[1]), i1 = norm_row_inv(pr, b[0], b[1]);
+        norm_apply_row(pr, m, i0, a, g, a_lds, lda, write_global);
+        norm_apply_row(pr, m + nw, i1, b, g, a_lds, lda, write_global);
+      } else {
+        norm_apply_row(pr, m, norm_row_inv(pr, a[0], a[1]), a, g, a_lds, lda, write_global);
+      }
+    };
+    if (m0 >= M) return;
+    rows(m0, x0, x1);
+    for (int m = m0 + 2 * nw; m < M; m += 2 * nw) {
+      v4i a[2], b[2];
+      norm_row_load(xr, (uint32_t)(m * pr.ldx * 2), nch, a);
+      norm_row_load(xr, (uint32_t)((m + nw) * pr.ldx * 2), nch, b);  // past row M - 1: zeros
+      rows(m, a, b);
+    }
+  }
+};
+
+// The i8 rows [M][K], loaded at kernel entry (16-byte chunks, PRE_CHUNKS per thread) and staged in LDS.
+constexpr int PRE_CHUNKS = 8;
+
+template <>
+struct NormStage<NORM_QUANT> {
+  v4i c[PRE_CHUNKS];
+
+  __device__ __forceinline__ void load(const NormQuant& pr, int M) {
+    const int nt = blockDim.x, tid = threadIdx.x, total = M * (pr.K >> 4);
+    const Rsrc q = rsrc(pr.hq_out, (int64_t)M * pr.K);
+#pragma unroll
+    for (int i = 0; i < PRE_CHUNKS; ++i) {
+      const int j = tid + i * nt;
+      c[i] = ld16(q, j < total ? 16 * j : LD_OOB);
+    }
+  }
+
+  __device__ __forceinline__ void store(const NormQuant& pr, int M, int8_t* a_lds, int lda, bool) {
+    const int nt = blockDim.x, tid = threadIdx.x, nch = pr.K >> 4, total = M * nch;
+#pragma unroll
+    for (int i = 0; i < PRE_CHUNKS; ++i) {
+      const int j = tid + i * nt;
+      if (j < total) *reinterpret_cast<v4i*>(a_lds + (j / nch) * lda + 16 * (j % nch)) = c[i];
+    }
+    // small workgroups: the chunks beyond the prefetched ones
+    const Rsrc q = rsrc(pr.hq_out, (int64_t)M * pr.K);
+    for (int j = tid + PRE_CHUNKS * nt; j < total; j += nt)
+      *reinterpret_cast<v4i*>(a_lds + (j / nch) * lda + 16 * (j % nch)) = ld16(q, 16 * j);
+  }
+};
 
 // the rows from m0 on
 __device__ __forceinline__ void norm_rows_from(NormQuant& pr, int64_t m0) {
@@ -580,7 +576,7 @@ __device__ __forceinline__ T pick3(int role, const T (&v)[3]) {
 // SPL > 1 (decode chain, no head norm): SPL workgroups per head block, workgroup s taking the
 // 16-column tiles t with t % SPL == s -- a tile and its RoPE partner t + D/32 fall in the same
 // workgroup when (D / 32) % SPL == 0 -- so each streams 1/SPL of the head's weights.
-template <int MAXW, bool RESID, int SPL = 1, int PFN = PF>
+template <int MAXW, bool RESID, int SPL = 1, int PFN = PF, int FORM = NORM_SHARED>
 __global__ __launch_bounds__(64 * MAXW) void attn_in_kernel(AttnInArgs p) {
   kernarg_warm<sizeof(AttnInArgs)>();
   extern __shared__ __attribute__((aligned(16))) int8_t dyn[];
@@ -619,16 +615,12 @@ __global__ __launch_bounds__(64 * MAXW) void attn_in_kernel(AttnInArgs p) {
     rp_own = ld4(rpr, tid < M ? 4 * tid : LD_OOB);
   }
   issue_fence();
-  const NormMap nm = norm_map(M);
-  NormRegs nr;
-  PreRows pq;
+  NormStage<FORM> ns;
   ResidRegs rr;
   if constexpr (RESID)
     resid_prefetch(p.pre, p.res, rr);
-  else if (p.pre.prequant)
-    prerows_load(p.pre, M, pq);
   else
-    norm_prefetch(p.pre, M, nm, nr);
+    ns.load(p.pre, M);
   issue_fence();
   const Rsrc wr = rsrc(pick3(role, p.W), (int64_t)Nrole * p.K);
   WSlice<PFN> ws;
@@ -655,10 +647,8 @@ __global__ __launch_bounds__(64 * MAXW) void attn_in_kernel(AttnInArgs p) {
   if constexpr (RESID) {
     if (b == 0) zero_rows(p.zero, p.zero_n);
     resid_norm_quant(p.pre, p.res, rr, a_lds, b == 0, red64);
-  } else if (p.pre.prequant) {
-    prerows_store(p.pre, M, pq, a_lds, lda);
   } else {
-    norm_quant_rows(p.pre, nr, M, nm, a_lds, lda, b == 0);
+    ns.store(p.pre, M, a_lds, lda, b == 0);
   }
   const int pos0 = p.pos_dev ? __builtin_amdgcn_readfirstlane(posv) : p.pos;
   const bool rows = p.row_pos != nullptr;
@@ -791,7 +781,7 @@ constexpr int WD_PF = 4;  // down-projection panel columns per thread loaded at 
 
 // BLK (more than 16 rows): workgroup (x, y) computes the rows 16 y .. 16 y + 15 alone, every row operand
 // and result moved on by 16 y rows.
-template <int MAXW, bool BLK = false>
+template <int MAXW, int FORM, bool BLK = false>
 __global__ __launch_bounds__(64 * MAXW) void mlp_in_kernel(MlpInArgs p) {
   kernarg_warm<sizeof(MlpInArgs)>();
   if constexpr (BLK) {
@@ -812,13 +802,8 @@ __global__ __launch_bounds__(64 * MAXW) void mlp_in_kernel(MlpInArgs p) {
   const int col = lane & 15, kg = lane >> 4;
   const int n = blockIdx.x * 16 + col;
 
-  const NormMap nm = norm_map(p.M);
-  NormRegs nr;
-  PreRows pq;
-  if (p.pre.prequant)
-    prerows_load(p.pre, p.M, pq);
-  else
-    norm_prefetch(p.pre, p.M, nm, nr);
+  NormStage<FORM> ns;
+  ns.load(p.pre, p.M);
   issue_fence();
   SigRegs sr;
   sig_prefetch(sr);
@@ -839,10 +824,7 @@ __global__ __launch_bounds__(64 * MAXW) void mlp_in_kernel(MlpInArgs p) {
   int32_t buv = ld4(rsrc(p.bu, (int64_t)p.N * 4), o4);
   issue_fence();
 
-  if (p.pre.prequant)
-    prerows_store(p.pre, p.M, pq, dyn, lda);
-  else
-    norm_quant_rows(p.pre, nr, p.M, nm, dyn, lda, blockIdx.x == 0);
+  ns.store(p.pre, p.M, dyn, lda, blockIdx.x == 0);
   sig_store(sr, sig32);
   __syncthreads();
   red[wave][lane] = wslice_mfma(ws, wr, dyn, lda, p.M, p.K);
@@ -1080,9 +1062,8 @@ struct NormGemvArgs {
   int ring_cap, vocab;
 };
 
-// (64 VGPRs: four workgroups of eight waves per CU; at 68 the 16-row head took 38.8 us, 34.9 at 64)
-template <int MAXW>
-__global__ __launch_bounds__(64 * MAXW, 4) void norm_gemv_kernel(NormGemvArgs p) {
+template <int MAXW, int FORM>
+__global__ __launch_bounds__(64 * MAXW) void norm_gemv_kernel(NormGemvArgs p) {
   kernarg_warm<sizeof(NormGemvArgs)>();
   extern __shared__ __attribute__((aligned(16))) int8_t dyn[];
   __shared__ v4i red[MAXW][64];
@@ -1095,13 +1076,8 @@ __global__ __launch_bounds__(64 * MAXW, 4) void norm_gemv_kernel(NormGemvArgs p)
 
   // the record slot of this decode launch (an earlier launch wrote it)
   int32_t stepv = ld4(rsrc(p.keys ? p.step : nullptr, 4), 0);
-  const NormMap nm = norm_map(p.M);
-  NormRegs nr;
-  PreRows pq;
-  if (p.pre.prequant)
-    prerows_load(p.pre, p.M, pq);
-  else
-    norm_prefetch(p.pre, p.M, nm, nr);
+  NormStage<FORM> ns;
+  ns.load(p.pre, p.M);
   issue_fence();
   SigRegs sr;
   sig_prefetch(sr);
@@ -1128,10 +1104,7 @@ __global__ __launch_bounds__(64 * MAXW, 4) void norm_gemv_kernel(NormGemvArgs p)
   }
   issue_fence();
 
-  if (p.pre.prequant)
-    prerows_store(p.pre, p.M, pq, dyn, lda);
-  else
-    norm_quant_rows(p.pre, nr, p.M, nm, dyn, lda, blockIdx.x == 0);
+  ns.store(p.pre, p.M, dyn, lda, blockIdx.x == 0);
   sig_store(sr, sig32);
   __syncthreads();
   v4i acc = wslice_mfma(ws, wr, dyn, lda, p.M, p.K);
@@ -1215,6 +1188,11 @@ extern "C" int llhip_rmsnorm_quant(const llhip_norm_quant_desc* d, int64_t M, vo
   return 0;
 }
 
+// the prologue form of M rows in workgroups of `waves` waves
+static int norm_form(const NormQuant& pr, int M, int waves) {
+  return pr.prequant ? NORM_QUANT : 2 * M <= waves ? NORM_SHARED : NORM_ROWS;
+}
+
 static int attn_in_args(const llhip_attn_in_desc* d, AttnInArgs& p, int& waves, size_t& lds, int min_threads) {
   if (!d) return fail(-EINVAL, "attn_in: null descriptor");
   int rc = fill_pre(p.pre, d->pre);
@@ -1275,13 +1253,13 @@ static int attn_in_args(const llhip_attn_in_desc* d, AttnInArgs& p, int& waves, 
   return 0;
 }
 
-template <bool RESID>
+template <bool RESID, int FORM = NORM_SHARED>
 static int attn_in_launch(const AttnInArgs& p, int waves, size_t lds, void* stream) {
   const dim3 grid((unsigned)(p.H + 2 * p.Hkv)), block(64 * waves);
   if (waves <= FUSED_WAVES)
-    hipLaunchKernelGGL((attn_in_kernel<FUSED_WAVES, RESID>), grid, block, lds, (hipStream_t)stream, p);
+    hipLaunchKernelGGL((attn_in_kernel<FUSED_WAVES, RESID, 1, PF, FORM>), grid, block, lds, (hipStream_t)stream, p);
   else
-    hipLaunchKernelGGL((attn_in_kernel<16, RESID>), grid, block, lds, (hipStream_t)stream, p);
+    hipLaunchKernelGGL((attn_in_kernel<16, RESID, 1, PF, FORM>), grid, block, lds, (hipStream_t)stream, p);
   LLHIP_LAUNCH_CHECK();
   return 0;
 }
@@ -1339,7 +1317,12 @@ extern "C" int llhip_attn_in(const llhip_attn_in_desc* d, void* stream) {
   int waves = 0;
   size_t lds = 0;
   const int rc = attn_in_args(d, p, waves, lds, 0);
-  return rc ? rc : attn_in_launch<false>(p, waves, lds, stream);
+  if (rc) return rc;
+  switch (norm_form(p.pre, p.M, waves)) {
+    case NORM_SHARED: return attn_in_launch<false, NORM_SHARED>(p, waves, lds, stream);
+    case NORM_ROWS: return attn_in_launch<false, NORM_ROWS>(p, waves, lds, stream);
+    default: return attn_in_launch<false, NORM_QUANT>(p, waves, lds, stream);
+  }
 }
 
 extern "C" int llhip_dec_attn_in(const llhip_attn_in_desc* d, const llhip_resid_desc* r, void* zero, int64_t zero_n,
@@ -1418,8 +1401,14 @@ extern "C" int llhip_mlp_in(const llhip_mlp_in_desc* d, void* stream) {
     const int nrc = llhip_rmsnorm_quant(&d->pre, d->M, stream);
     if (nrc) return nrc;
   }
-  hipLaunchKernelGGL((mlp_in_kernel<FUSED_WAVES>), dim3((unsigned)ceil_div(p.N, 16)), dim3(128 * p.KS),
-                     (size_t)(p.M * (p.K + 16)), (hipStream_t)stream, p);
+  const dim3 grid((unsigned)ceil_div(p.N, 16)), block(128 * p.KS);
+  const size_t lds = (size_t)(p.M * (p.K + 16));
+  hipStream_t s = (hipStream_t)stream;
+  switch (norm_form(p.pre, p.M, 2 * p.KS)) {
+    case NORM_SHARED: hipLaunchKernelGGL((mlp_in_kernel<FUSED_WAVES, NORM_SHARED>), grid, block, lds, s, p); break;
+    case NORM_ROWS: hipLaunchKernelGGL((mlp_in_kernel<FUSED_WAVES, NORM_ROWS>), grid, block, lds, s, p); break;
+    default: hipLaunchKernelGGL((mlp_in_kernel<FUSED_WAVES, NORM_QUANT>), grid, block, lds, s, p); break;
+  }
   LLHIP_LAUNCH_CHECK();
   return 0;
 }
@@ -1440,8 +1429,13 @@ extern "C" int llhip_mlp_in_blocks(const llhip_mlp_in_desc* d, void* stream) {
   if (rc) return rc;
   p.M = (int)d->M;
   if (apart && (rc = llhip_rmsnorm_quant(&d->pre, d->M, stream))) return rc;
-  hipLaunchKernelGGL((mlp_in_kernel<FUSED_WAVES, true>), dim3((unsigned)ceil_div(p.N, 16), (unsigned)blocks),
-                     dim3(128 * p.KS), (size_t)(dd.M * (p.K + 16)), (hipStream_t)stream, p);
+  const dim3 grid((unsigned)ceil_div(p.N, 16), (unsigned)blocks), block(128 * p.KS);
+  const size_t lds = (size_t)(dd.M * (p.K + 16));
+  hipStream_t s = (hipStream_t)stream;
+  if (p.pre.prequant)
+    hipLaunchKernelGGL((mlp_in_kernel<FUSED_WAVES, NORM_QUANT, true>), grid, block, lds, s, p);
+  else  // (the last block's rows may be few: NORM_ROWS takes any number)
+    hipLaunchKernelGGL((mlp_in_kernel<FUSED_WAVES, NORM_ROWS, true>), grid, block, lds, s, p);
   LLHIP_LAUNCH_CHECK();
   return 0;
 }
@@ -1532,9 +1526,14 @@ static int norm_linear_args(const llhip_norm_linear_desc* d, NormGemvArgs& p, in
 }
 
 static int norm_linear_launch(const NormGemvArgs& p, void* stream) {
-  const int blocks = (int)ceil_div(ceil_div(p.N, 16), p.TPW);
-  hipLaunchKernelGGL((norm_gemv_kernel<FUSED_WAVES>), dim3((unsigned)blocks), dim3(64 * p.TPW * p.KS),
-                     (size_t)(p.M * (p.K + 16)), (hipStream_t)stream, p);
+  const dim3 grid((unsigned)ceil_div(ceil_div(p.N, 16), p.TPW)), block(64 * p.TPW * p.KS);
+  const size_t lds = (size_t)(p.M * (p.K + 16));
+  hipStream_t s = (hipStream_t)stream;
+  switch (norm_form(p.pre, p.M, p.TPW * p.KS)) {
+    case NORM_SHARED: hipLaunchKernelGGL((norm_gemv_kernel<FUSED_WAVES, NORM_SHARED>), grid, block, lds, s, p); break;
+    case NORM_ROWS: hipLaunchKernelGGL((norm_gemv_kernel<FUSED_WAVES, NORM_ROWS>), grid, block, lds, s, p); break;
+    default: hipLaunchKernelGGL((norm_gemv_kernel<FUSED_WAVES, NORM_QUANT>), grid, block, lds, s, p); break;
+  }
   LLHIP_LAUNCH_CHECK();
   return 0;
 }

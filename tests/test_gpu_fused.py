@@ -225,3 +225,87 @@ def test_rows_normalised_in_the_prologue(M, K, N):
     for a, b in zip(*outs):
         assert np.array_equal(a, b)
     assert np.abs(outs[0][4]).max() > 0
+
+
+@pytest.mark.parametrize("K,H,Hkv,D,norm", [(64, 4, 2, 16, 0), (576, 9, 3, 64, 0), (896, 14, 2, 64, 0), (1024, 4, 2, 128, 1),
+                                            (768, 4, 2, 256, 1)])
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 9, 12, 13, 16])
+def test_attn_in_rows_normalised_in_the_prologue(M, K, H, Hkv, D, norm):
+    """llhip_attn_in of one to 16 rows normalising them itself (one wave per workgroup up to sixteen, several waves
+    to a row, one wave to one, two or more rows) writes what llhip_rmsnorm_quant followed by the prequantised
+    form writes, rows at positions of their own."""
+    import ctypes
+
+    from llaccel_amd import _lib
+    from tests.gpu_helpers import ptr, random_rq, stream, torch, up
+
+    t = torch()
+    rng = np.random.default_rng(100 * M + K)
+    max_seq = 64
+    x, g = up(rng.integers(-32768, 32768, (M, K)), np.int16), up(rng.integers(-32768, 32768, K), np.int16)
+    cols = (H * D, Hkv * D, Hkv * D)
+    w = [up(rng.integers(-127, 128, (n, K)), np.int8) for n in cols]
+    rq = [up(random_rq(rng, n, K, i == 2), np.int32) for i, n in enumerate(cols)]
+    hg = [up(rng.integers(-32768, 32768, D), np.int16) for _ in range(2)]
+    tab = [up(rng.integers(-16384, 16385, (max_seq, D // 2)), np.int16) for _ in range(2)]
+    pos = up(rng.permutation(max_seq)[:M], np.int32)
+    outs = []
+    for pre in (0, 1):
+        def z(*shape, dt=t.int16):
+            return t.zeros(shape, dtype=dt, device="cuda")
+
+        h, hq = z(M, K), z(M, K, dt=t.int8)
+        lin = [z(M, n, dt=t.int8 if i == 2 else t.int16) for i, n in enumerate(cols)]
+        nrm, rope, quant = ([z(M, n, dt=dt) for n in cols[:2]] for dt in (t.int16, t.int16, t.int8))
+        kc, vc = (z(M, Hkv, max_seq, D, dt=t.int8) for _ in range(2))
+        d = _lib.AttnInDesc()
+        n = d.pre
+        n.x, n.gamma, n.h_out, n.hq_out, n.ldx, n.K = ptr(x), ptr(g), ptr(h), ptr(hq), K, K
+        n.eps_t, n.C, n.sh_post, n.Mq, n.Sq, n.prequant = 999, int(2**24 * K**0.5), 24, 1234567891, 38, pre
+        for i in range(3):
+            d.W[i], d.rq[i], d.bias[i], d.lin_out[i] = ptr(w[i]), ptr(rq[i]), None, ptr(lin[i])
+        for i in range(2):
+            d.nrm_gamma[i], d.nrm_out[i] = ptr(hg[i]), ptr(nrm[i])
+            d.nrm_eps[i], d.nrm_C[i], d.nrm_sh[i] = 99, int(2**22 * D**0.5), 22
+            d.rope_out[i], d.quant_out[i], d.quant_M[i], d.quant_S[i] = ptr(rope[i]), ptr(quant[i]), 1234567891, 38
+        d.cos_tab, d.sin_tab, d.row_pos, d.slot_stride = ptr(tab[0]), ptr(tab[1]), ptr(pos), Hkv * max_seq * D
+        d.kc, d.vc, d.max_seq, d.M, d.H, d.Hkv, d.D, d.has_norm = ptr(kc), ptr(vc), max_seq, M, H, Hkv, D, norm
+        if pre:
+            _lib.call("llhip_rmsnorm_quant", ctypes.byref(n), M, stream())
+        _lib.call("llhip_attn_in", ctypes.byref(d), stream())
+        outs.append([a.cpu().numpy() for a in (h, hq, *lin, *nrm, *rope, *quant, kc, vc)])
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
+    assert np.abs(outs[0][1]).max() > 0 and np.abs(outs[0][-1]).max() > 0
+
+
+@pytest.mark.parametrize("K,N", [(64, 256), (576, 1040), (896, 65600)])
+@pytest.mark.parametrize("M", [1, 2, 4, 5, 8, 16])
+def test_norm_linear_rows_normalised_in_the_prologue(M, K, N):
+    """llhip_norm_linear in its three forms of the rows (few and many tiles per workgroup): one launch writes what
+    llhip_rmsnorm_quant followed by the prequantised form writes."""
+    import ctypes
+
+    from llaccel_amd import _lib
+    from tests.gpu_helpers import ptr, random_rq, stream, torch, up
+
+    t = torch()
+    rng = np.random.default_rng(100 * M + K)
+    x, g = up(rng.integers(-32768, 32768, (M, K)), np.int16), up(rng.integers(-32768, 32768, K), np.int16)
+    w, rq = up(rng.integers(-127, 128, (N, K)), np.int8), up(random_rq(rng, N, K, False), np.int32)
+    outs = []
+    for pre in (0, 1):
+        h, hq = t.zeros((M, K), dtype=t.int16, device="cuda"), t.zeros((M, K), dtype=t.int8, device="cuda")
+        out = t.zeros((M, N), dtype=t.int16, device="cuda")
+        d = _lib.NormLinearDesc()
+        n = d.pre
+        n.x, n.gamma, n.h_out, n.hq_out, n.ldx, n.K = ptr(x), ptr(g), ptr(h), ptr(hq), K, K
+        n.eps_t, n.C, n.sh_post, n.Mq, n.Sq, n.prequant = 999, int(2**24 * K**0.5), 24, 1234567891, 38, pre
+        d.W, d.rq, d.out, d.M, d.N, d.silu_Mi, d.silu_Si, d.silu_sh = ptr(w), ptr(rq), ptr(out), M, N, 1 << 30, 30, 16
+        if pre:
+            _lib.call("llhip_rmsnorm_quant", ctypes.byref(n), M, stream())
+        _lib.call("llhip_norm_linear", ctypes.byref(d), stream())
+        outs.append([a.cpu().numpy() for a in (h, hq, out)])
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
+    assert np.abs(outs[0][2]).max() > 0
