@@ -1193,6 +1193,17 @@ static int norm_form(const NormQuant& pr, int M, int waves) {
   return pr.prequant ? NORM_QUANT : 2 * M <= waves ? NORM_SHARED : NORM_ROWS;
 }
 
+// Waves of a workgroup whose GEMM uses `waves` of them: more, up to FUSED_WAVES, while it normalises more
+// rows than it has waves (a wave's rows are a serial chain of which two overlap) and every workgroup has a
+// CU of its own.  The waves past the GEMM's have no K steps.  Before / after (us): attn_in of 64 columns (one
+// wave) 4 rows 6.9 / 4.9, 16 rows 16.2 / 6.6 (7.0 with a launch of their own); mlp_in of 64 (two waves) 8 rows 7.9 /
+// 6.05, 16 rows 10.8 / 7.0 (6.7); with more workgroups than CUs a loss, 5 rows of FFN 4864 of 896 (four) 7.7 / 8.3.
+static int norm_waves(const NormQuant& pr, int M, int waves, int64_t workgroups) {
+  if (!pr.prequant && M > 1 && workgroups <= current_cu_count())
+    while (waves < M && 2 * waves <= FUSED_WAVES) waves *= 2;
+  return waves;
+}
+
 static int attn_in_args(const llhip_attn_in_desc* d, AttnInArgs& p, int& waves, size_t& lds, int min_threads) {
   if (!d) return fail(-EINVAL, "attn_in: null descriptor");
   int rc = fill_pre(p.pre, d->pre);
@@ -1318,6 +1329,15 @@ extern "C" int llhip_attn_in(const llhip_attn_in_desc* d, void* stream) {
   size_t lds = 0;
   const int rc = attn_in_args(d, p, waves, lds, 0);
   if (rc) return rc;
+  // Thirteen rows and more of 512 < K < 640: normalised by a launch of their own (such a row costs a second
+  // pass of the wave for at most 16 of its lanes; of 576, 13 rows 7.8 us in the prologue, 7.65 in two launches,
+  // 16 rows 8.2 / 7.7; of 640 and more no difference or a gain, 16 rows of 896 8.0 / 8.3)
+  if (d->M > 12 && !p.pre.prequant && p.pre.hq_out && waves <= FUSED_WAVES && p.K > 512 && p.K < 640) {
+    const int nrc = llhip_rmsnorm_quant(&d->pre, d->M, stream);
+    if (nrc) return nrc;
+    p.pre.prequant = 1;
+  }
+  waves = norm_waves(p.pre, p.M, waves, p.H + 2 * p.Hkv);
   switch (norm_form(p.pre, p.M, waves)) {
     case NORM_SHARED: return attn_in_launch<false, NORM_SHARED>(p, waves, lds, stream);
     case NORM_ROWS: return attn_in_launch<false, NORM_ROWS>(p, waves, lds, stream);
@@ -1386,25 +1406,24 @@ static int mlp_in_args(const llhip_mlp_in_desc* d, MlpInArgs& p, int min_threads
 }
 
 extern "C" int llhip_mlp_in(const llhip_mlp_in_desc* d, void* stream) {
-  if (!d) return fail(-EINVAL, "mlp_in: null descriptor");
-  // More than 8 rows and more workgroups than CUs (two prologues on some CUs): the rows normalised
-  // once, in a launch of their own.  16 rows of 896, FFN 4864 (304 workgroups): 12.2 us with the rows
-  // normalised in every workgroup against 8.3 + 2.9 us; FFN 1536 (96 workgroups) 12 rows 6.5 against
-  // 6.4 + 2.5 us, and 8 rows of FFN 4864 gain too.
-  llhip_mlp_in_desc dd = *d;
-  const bool apart = !d->pre.prequant && d->M > 8 && d->pre.hq_out && ceil_div(d->N, 16) > current_cu_count();
-  if (apart) dd.pre.prequant = 1;
   MlpInArgs p{};
-  const int rc = mlp_in_args(&dd, p, 0);
+  int rc = mlp_in_args(d, p, 0);
   if (rc) return rc;
-  if (apart) {
-    const int nrc = llhip_rmsnorm_quant(&d->pre, d->M, stream);
-    if (nrc) return nrc;
+  // The rows normalised by a launch of their own from 8 rows on with more workgroups than CUs (two prologues
+  // on some CUs).  In the prologue / in two launches (us): FFN 4864 of 896, 7 rows 8.1 / 8.4, 8 rows 8.7 / 8.35, 16
+  // rows 12.2 / 8.2; FFN 1536 of 576 (96 workgroups) 12 rows 6.9 / 7.7.
+  if (d->M >= 8 && !p.pre.prequant && p.pre.hq_out && ceil_div(p.N, 16) > current_cu_count()) {
+    llhip_mlp_in_desc dd = *d;
+    dd.pre.prequant = 1;
+    rc = mlp_in_args(&dd, p, 0);
+    if (!rc) rc = llhip_rmsnorm_quant(&d->pre, d->M, stream);
+    if (rc) return rc;
   }
-  const dim3 grid((unsigned)ceil_div(p.N, 16)), block(128 * p.KS);
+  const int waves = norm_waves(p.pre, p.M, 2 * p.KS, ceil_div(p.N, 16));
+  const dim3 grid((unsigned)ceil_div(p.N, 16)), block(64 * waves);
   const size_t lds = (size_t)(p.M * (p.K + 16));
   hipStream_t s = (hipStream_t)stream;
-  switch (norm_form(p.pre, p.M, 2 * p.KS)) {
+  switch (norm_form(p.pre, p.M, waves)) {
     case NORM_SHARED: hipLaunchKernelGGL((mlp_in_kernel<FUSED_WAVES, NORM_SHARED>), grid, block, lds, s, p); break;
     case NORM_ROWS: hipLaunchKernelGGL((mlp_in_kernel<FUSED_WAVES, NORM_ROWS>), grid, block, lds, s, p); break;
     default: hipLaunchKernelGGL((mlp_in_kernel<FUSED_WAVES, NORM_QUANT>), grid, block, lds, s, p); break;
@@ -1415,21 +1434,23 @@ extern "C" int llhip_mlp_in(const llhip_mlp_in_desc* d, void* stream) {
 
 extern "C" int llhip_mlp_in_blocks(const llhip_mlp_in_desc* d, void* stream) {
   if (!d) return fail(-EINVAL, "mlp_in: null descriptor");
-  int rc = 0;
   if (d->M < 1 || d->M > LLHIP_BLOCK_ROWS_MAX) return fail(-EINVAL, "mlp_in: 1 to %d rows", LLHIP_BLOCK_ROWS_MAX);
-  if (d->M * d->pre.ldx >= (1ll << 30)) return fail(-EINVAL, "mlp_in: rows above 2 GiB");
-  // the rows normalised once when there are more workgroups than CUs, as in llhip_mlp_in
-  llhip_mlp_in_desc dd = *d;
+  if (d->pre.ldx >= (1ll << 30) / d->M) return fail(-EINVAL, "mlp_in: rows above 2 GiB");
   const int64_t blocks = ceil_div(d->M, 16);
-  const bool apart = !d->pre.prequant && d->pre.hq_out && ceil_div(d->N, 16) * blocks > current_cu_count();
-  if (apart) dd.pre.prequant = 1;
+  llhip_mlp_in_desc dd = *d;
   dd.M = std::min<int64_t>(d->M, 16);
   MlpInArgs p{};
-  rc = mlp_in_args(&dd, p, 0);
+  int rc = mlp_in_args(&dd, p, 0);
   if (rc) return rc;
+  // the rows normalised by a launch of their own when there are more workgroups than CUs, as in llhip_mlp_in
+  if (!p.pre.prequant && p.pre.hq_out && ceil_div(p.N, 16) * blocks > current_cu_count()) {
+    dd.pre.prequant = 1;
+    rc = mlp_in_args(&dd, p, 0);
+    if (!rc) rc = llhip_rmsnorm_quant(&d->pre, d->M, stream);
+    if (rc) return rc;
+  }
   p.M = (int)d->M;
-  if (apart && (rc = llhip_rmsnorm_quant(&d->pre, d->M, stream))) return rc;
-  const dim3 grid((unsigned)ceil_div(p.N, 16), (unsigned)blocks), block(128 * p.KS);
+  const dim3 grid((unsigned)ceil_div(p.N, 16), (unsigned)blocks), block(64 * norm_waves(p.pre, (int)dd.M, 2 * p.KS, blocks * ceil_div(p.N, 16)));
   const size_t lds = (size_t)(dd.M * (p.K + 16));
   hipStream_t s = (hipStream_t)stream;
   if (p.pre.prequant)

@@ -309,3 +309,43 @@ def test_norm_linear_rows_normalised_in_the_prologue(M, K, N):
     for a, b in zip(*outs):
         assert np.array_equal(a, b)
     assert np.abs(outs[0][2]).max() > 0
+
+
+@pytest.mark.parametrize("K,N", [(64, 192), (128, 400), (896, 4128)])
+@pytest.mark.parametrize("M", [4, 5, 7, 8, 12, 13, 16, 17, 40])
+def test_waves_of_the_prologue(M, K, N):
+    """Workgroups whose GEMM takes two and four waves, with more of them for the rows, and the rows in a launch of their own:
+    eight rows and more with more workgroups than compute units."""
+    test_rows_normalised_in_the_prologue(M, K, N)
+
+
+def test_rows_normalised_without_quantised_rows_out():
+    """Without hq_out the rows cannot come from a launch of their own: they are normalised in the workgroups."""
+    import ctypes
+
+    from llaccel_amd import _lib
+    from tests.gpu_helpers import ptr, random_rq, stream, torch, up
+
+    t = torch()
+    rng = np.random.default_rng(5)
+    M, K, N = 16, 64, 4128
+    x, g = up(rng.integers(-32768, 32768, (M, K)), np.int16), up(rng.integers(-32768, 32768, K), np.int16)
+    wg, wu = (up(rng.integers(-127, 128, (N, K)), np.int8) for _ in range(2))
+    rqg, rqu = (up(random_rq(rng, N, K, False), np.int32) for _ in range(2))
+    outs = []
+    for out in (True, False):
+        hq = t.zeros((M, K), dtype=t.int8, device="cuda") if out else None
+        sg, f = (t.zeros((M, N), dtype=t.int16, device="cuda") for _ in range(2))
+        fq = t.zeros((M, N), dtype=t.int8, device="cuda")
+        d = _lib.MlpInDesc()
+        n = d.pre
+        n.x, n.gamma, n.h_out, n.hq_out, n.ldx, n.K = ptr(x), ptr(g), None, ptr(hq), K, K
+        n.eps_t, n.C, n.sh_post, n.Mq, n.Sq, n.prequant = 999, int(2**24 * K**0.5), 24, 1234567891, 38, 0
+        d.Wg, d.Wu, d.rqg, d.rqu = ptr(wg), ptr(wu), ptr(rqg), ptr(rqu)
+        d.sg_out, d.f_out, d.fq_out = ptr(sg), ptr(f), ptr(fq)
+        d.silu_Mi, d.silu_Si, d.silu_sh, d.mul_sh, d.fq_M, d.fq_S, d.M, d.N = 1 << 30, 30, 16, 11, 1 << 30, 37, M, N
+        _lib.call("llhip_mlp_in", ctypes.byref(d), stream())
+        outs.append([a.cpu().numpy() for a in (sg, f, fq)])
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
+    assert np.abs(outs[0][2]).max() > 0
