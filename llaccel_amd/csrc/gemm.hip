@@ -35,7 +35,14 @@ struct LinearArgs {
   const int16_t* aux;
   void* out;
   int64_t lda, ldaux, ldo;
-  int64_t Mi;
+  union {
+    int64_t Mi;  // EPI_SILU
+    // EPI_ADD, the linear and add of an unfused graph (linear_gemv, linear_gemv1): the linear's own
+    // output rows (stride ldo), kept beside the sum; the add's shift of them is aux_shift.  (A field of
+    // its own costs every linear_mfma instance two scalar registers, and <0, *, 64, 128, 4, 128, 2>
+    // then spills to scratch.)
+    int16_t* pre;
+  };
   int M, K, N;
   int aux_shift, Si, sh;
   int steps;  // ceil(K / 64)
@@ -43,9 +50,6 @@ struct LinearArgs {
   int nfast;   // linear_mfma: tiles in N-fastest order (N-block l % nblk), else M-fastest
   int nblk;
   int mgroup;  // M-fastest order within groups of mgroup M-blocks (0: one group of all)
-  // EPI_ADD, the linear and add of an unfused graph (linear_gemv, linear_gemv1): the linear's own
-  // output rows (stride ldo), kept beside the sum; the add's shift of them is aux_shift
-  int16_t* pre;
 };
 
 // M-block and N-block of logical tile l: N-block fastest (nfast), or M-block fastest within groups
@@ -142,7 +146,7 @@ constexpr int GEMV_PF = 8;  // K steps of W and A in flight per wave
 
 template <int EPI, bool OUT8, bool ALIGNED>
 __global__ __launch_bounds__(64 * GEMV_MAX_WAVES) void linear_gemv(LinearArgs p) {
-  kernarg_warm<sizeof(LinearArgs)>();
+  kernarg_warm<sizeof(LinearArgs) + 16>();  // and the block size behind them (another line: 3 % of a short launch)
   __shared__ v4i red[GEMV_MAX_WAVES - 1][64];
   const int lane = threadIdx.x & 63;
   const int wave = wave_id();

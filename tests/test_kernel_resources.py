@@ -77,3 +77,10 @@ def test_eight_wave_workgroups_fit_twice(kernels):
         for n, k in _named(kernels, name).items():
             if k[".max_flat_workgroup_size"] <= 512:
                 assert k[".vgpr_count"] <= 128, (n, k[".vgpr_count"])
+
+
+def test_gemm_tiles_without_scratch(kernels):
+    """linear_mfma below the 256 x 256 tile: a vector register or an argument more sends the 64 x 128 instances to scratch."""
+    for n, k in _named(kernels, "linear_mfma").items():
+        if "ILi256E" not in n and "ELi256ELi256E" not in n:
+            assert k[".private_segment_fixed_size"] == 0, n
