@@ -143,8 +143,11 @@ __device__ __forceinline__ void finish_pre(const LinearArgs& p, const EpiOperand
 }
 
 constexpr int GEMV_PF = 8;  // K steps of W and A in flight per wave
+constexpr int GEMV_U = 4;   // and in the loop past them
 
-template <int EPI, bool OUT8, bool ALIGNED>
+// SPARSE: the steps of a group of loads past the wave's last one are left out, a uniform branch per step.
+// (A load costs its issue also where it reads nothing, a branch where there is nothing to leave out.)
+template <int EPI, bool OUT8, bool ALIGNED, bool SPARSE>
 __global__ __launch_bounds__(64 * GEMV_MAX_WAVES) void linear_gemv(LinearArgs p) {
   kernarg_warm<sizeof(LinearArgs) + 16>();  // and the block size behind them (another line: 3 % of a short launch)
   __shared__ v4i red[GEMV_MAX_WAVES - 1][64];
@@ -186,13 +189,23 @@ __global__ __launch_bounds__(64 * GEMV_MAX_WAVES) void linear_gemv(LinearArgs p)
       a = s < s_end ? load16_bytes(arow, k, p.K, avalid) : v4i{0, 0, 0, 0};
     }
   };
+  auto load_steps = [&](int s, auto& b, auto& a) {  // steps s .. s + N - 1
+    constexpr int N = sizeof(b) / sizeof(b[0]);
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      if (SPARSE && u > 0) {
+        b[u] = a[u] = v4i{0, 0, 0, 0};
+        if (s + u >= s_end) continue;
+      }
+      load(s + u, b[u], a[u]);
+    }
+  };
   v4i acc = {0, 0, 0, 0};
   int s = s_begin;
   // first GEMV_PF steps: every load issued before the first MFMA
   {
     v4i b[GEMV_PF], a[GEMV_PF];
-#pragma unroll
-    for (int u = 0; u < GEMV_PF; ++u) load(s + u, b[u], a[u]);
+    load_steps(s, b, a);
     EpiOperands<EPI> e{};
     if (wave == 0) {
       e.rq_m = p.rq[2 * nn];
@@ -209,11 +222,10 @@ __global__ __launch_bounds__(64 * GEMV_MAX_WAVES) void linear_gemv(LinearArgs p)
 #pragma unroll
     for (int u = 0; u < GEMV_PF; ++u) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[u], b[u], acc, 0, 0, 0);
     s += GEMV_PF;
-    constexpr int U = 4;
+    constexpr int U = GEMV_U;
     for (; s < s_end; s += U) {
       v4i bb[U], aa[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) load(s + u, bb[u], aa[u]);
+      load_steps(s, bb, aa);
 #pragma unroll
       for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(aa[u], bb[u], acc, 0, 0, 0);
     }
@@ -1677,10 +1689,20 @@ static int launch_linear(LinearArgs& p, void* ws, hipStream_t stream, const Norm
     nw = (int)std::min<int64_t>(GEMV_MAX_WAVES, ceil_div(p.steps, GEMV_PF));
   }
   dim3 grid((unsigned)ceil_div(p.N, p.cpb), 1, zblocks);
-  if (aligned && 16 * p.lda < (1ll << 31))  // 16 rows of A within a buffer's range
-    hipLaunchKernelGGL((linear_gemv<EPI, OUT8, true>), grid, dim3(64 * nw), 0, stream, p);
+  // Launches of many waves whose K ranges leave part of a group of loads empty skip it; a launch of few
+  // waves is one round trip of loads, which the branches only lengthen.  Without / with the branches (us):
+  // 2 x 896 x 4864 (1216 waves of four steps) 3.83 / 3.40, 2 x 896 x 151936 (fourteen steps) 26.1 / 24.0, 64 x
+  // 576 x 576 (576 waves of five) 3.22 / 3.09, 2 x 576 x 576 (288 waves of five) 2.75 / 2.94, 2 x 1024 x 32000 (sixteen
+  // steps, nothing to skip) 7.1 / 7.3.
+  const int spw = (int)ceil_div(p.steps, nw);
+  const bool partial = spw < GEMV_PF || (spw - GEMV_PF) % GEMV_U != 0;
+  const bool sparse = partial && (int64_t)grid.x * zblocks * nw > 2 * cus;
+  if (!aligned || 16 * p.lda >= (1ll << 31))  // (16 rows of A within a buffer's range)
+    hipLaunchKernelGGL((linear_gemv<EPI, OUT8, false, false>), grid, dim3(64 * nw), 0, stream, p);
+  else if (sparse)
+    hipLaunchKernelGGL((linear_gemv<EPI, OUT8, true, true>), grid, dim3(64 * nw), 0, stream, p);
   else
-    hipLaunchKernelGGL((linear_gemv<EPI, OUT8, false>), grid, dim3(64 * nw), 0, stream, p);
+    hipLaunchKernelGGL((linear_gemv<EPI, OUT8, true, false>), grid, dim3(64 * nw), 0, stream, p);
   LLHIP_LAUNCH_CHECK();
   return 0;
 }

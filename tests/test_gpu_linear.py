@@ -372,3 +372,17 @@ def test_linear_norm_equals_linear_then_rmsnorm_quant(M, K, N):
     with pytest.raises(ValueError):
         _lib.call("llhip_linear_norm", ptr(ad), M, K, K, ptr(wd), N, ptr(rqd), ptr(bd), ptr(auxd), N, ptr(xd), N,
                   ctypes.byref(d), ptr(workspace()), stream())
+
+
+@pytest.mark.parametrize("epilogue", ["none", "resadd"])
+@pytest.mark.parametrize("M,K,N", [(2, 896, 4864), (16, 592, 9000), (3, 64, 9001), (1, 80, 17000), (64, 576, 576), (16, 1040, 4100),
+                                   (33, 1536, 576)])
+def test_partial_groups_of_loads(M, K, N, epilogue):
+    """Launches of many waves whose K ranges end inside a group of loads: two steps to thirteen, a last wave of fewer, K
+    that ends inside a step, ragged N and rows."""
+    rng = np.random.default_rng(M + K + N)
+    a, w, rq = _operands(rng, M, K, N, out_i8=False)
+    bias = rng.integers(-3000, 3000, N)
+    aux = rng.integers(-32768, 32768, (M, N)) if epilogue == "resadd" else None
+    got = gpu_linear(a, w, rq, bias=bias, out_i8=False, epilogue=epilogue, aux=aux)
+    assert np.array_equal(got, O.linear_c(a, w, rq, bias, False, epilogue, aux, 0, None))
