@@ -1620,8 +1620,26 @@ static int launch_mfma_shape(LinearArgs& p, void* ws, hipStream_t stream, const 
   return launch_mfma<EPI, OUT8, 64, 128, 4, KT>(p, ws, stream, norm, norm_done);
 }
 
-static bool rows_in_blocks16(const LinearArgs& p, bool aligned) {
-  return p.M <= 1024 && aligned && p.K <= 3072 && ceil_div(p.M, 16) * (int64_t)p.N * p.K <= (16ll << 20);
+// More than 16 rows: the 16-row kernel over blocks of 16 rows (blockIdx.z) while re-reading W once per block
+// stays cheap (16 MiB) -- every load of a workgroup is requested at entry, so it is one memory round trip
+// where an LDS ring is one per few K tiles -- and while its workgroups are few beside what the other kernel
+// costs.  Time of the 16-row blocks over that of the tiles, measured:
+//  * K % 64 != 0 (linear_tiled): 100 x 592 x 3000 0.37, no bound needed;
+//  * K % 64 == 0 (64-byte K tiles): eight workgroups per CU 0.92 (K = 64), 0.86 (192), 0.95 (448), 16 1.3; with an
+//    epilogue 9 0.92 to 0.96, 12 1.2;
+//  * K % 128 == 0: K = 128 5 per CU 0.91, 8 1.02; 256 5 0.95, 6 1.01; 512 3 0.88, 4 0.99, 5 1.06; 768 3 0.89, 4 1.02;
+//    1024 3 0.90, 3.25 1.04; with an epilogue to 1.4 times as many: 256 8 1.0; 512 5 0.94, 6 1.04; 1024 4 0.96;
+//  * a tile has 64 rows: where the last is partly empty as many more (32 x 192 x 24000 with a residual add, 3000
+//    workgroups, 5.5 / 6.7 us).
+// 64 x 576 x 576 takes 3.1 us (5.6 in tiles), 64 x 3072 x 1024 5.5 (7.8), 32 x 4864 x 896 9.7 (8.7: past K = 3072 a
+// wave's chain is too long).
+static bool rows_in_blocks16(const LinearArgs& p, bool aligned, bool plain) {
+  const int64_t mb = ceil_div(p.M, 16), wgs = mb * ceil_div(p.N, 16), cus = current_cu_count();
+  if (p.M > 1024 || !aligned || p.K > 3072 || mb * p.N * p.K > (16ll << 20)) return false;
+  if (p.K % 64) return true;
+  const int64_t per_cu100 = std::max<int64_t>(340000 / (p.K + 320), 300);  // workgroups per CU, in hundredths
+  const int64_t most = p.K % 128 ? (plain ? 800 : 1000) : (plain ? per_cu100 : 7 * per_cu100 / 5);
+  return 100 * wgs * mb <= most * cus * 4 * ceil_div(p.M, 64);
 }
 static bool linear_aligned(const LinearArgs& p) {
   return p.K % 16 == 0 && p.lda % 16 == 0 && (uintptr_t)p.A % 16 == 0 && (uintptr_t)p.W % 16 == 0;
@@ -1631,15 +1649,9 @@ template <int EPI, bool OUT8>
 static int launch_linear(LinearArgs& p, void* ws, hipStream_t stream, const NormQuant* norm = nullptr,
                          bool* norm_done = nullptr) {
   const bool aligned = linear_aligned(p);
-  // More than 16 rows: the 16-row kernel over blocks of 16 rows (blockIdx.z) while re-reading W once
-  // per block stays cheap -- every load of a workgroup is requested at entry, so it is one memory
-  // round trip where an LDS ring is one per few K tiles.  Measured (us, 16-row blocks / MFMA tiles):
-  // 64 x 576 x 576 3.3 / 5.6, 64 x 3072 x 1024 5.5 / 7.8, 256 x 896 x 896 5.8 / 6.2, 400 x 576 x 576
-  // 3.9 / 6.0 (ceil(M/16) N K at most 16 MiB), against 400 x 896 x 896 7.4 / 6.5, 64 x 896 x 4864
-  // 7.0 / 6.1 (17 MB and more), 32 x 4864 x 896 9.7 / 8.7 (K past 3072: long serial chains per wave).
   // Rows that are normalised next (norm) keep the MFMA tiles where those split K (from K = 1024 on):
   // their finishing launch normalises too, which saves a launch.
-  const bool blocks16 = p.M > 16 && rows_in_blocks16(p, aligned) && (!norm || p.K < 1024);
+  const bool blocks16 = p.M > 16 && rows_in_blocks16(p, aligned, EPI == EPI_NONE) && (!norm || p.K < 1024);
   if constexpr (EPI != EPI_ADD) {  // (llhip_linear_add comes here with rows of the kernels below only)
     if (p.M > 16 && p.K % 64 == 0 && aligned && !blocks16) {
       if (p.K % 128 == 0) return launch_mfma_shape<EPI, OUT8, 128>(p, ws, stream, norm, norm_done);
@@ -1849,7 +1861,7 @@ extern "C" int llhip_linear_add(const int8_t* A, int64_t M, int64_t K, int64_t l
   hipStream_t s = (hipStream_t)stream;
   // one launch where the 16-row kernels run: their epilogue keeps both rows
   const bool aligned = linear_aligned(p);
-  if (M <= 16 || rows_in_blocks16(p, aligned)) {
+  if (M <= 16 || rows_in_blocks16(p, aligned, false)) {
     p.pre = o;
     p.aux_shift = (int)sh_b;
     return launch_linear<EPI_ADD, false>(p, ws, s);

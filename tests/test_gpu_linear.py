@@ -386,3 +386,15 @@ def test_partial_groups_of_loads(M, K, N, epilogue):
     aux = rng.integers(-32768, 32768, (M, N)) if epilogue == "resadd" else None
     got = gpu_linear(a, w, rq, bias=bias, out_i8=False, epilogue=epilogue, aux=aux)
     assert np.array_equal(got, O.linear_c(a, w, rq, bias, False, epilogue, aux, 0, None))
+
+
+@pytest.mark.parametrize("epilogue", ["none", "resadd"])
+@pytest.mark.parametrize("M,K,N", [(1024, 64, 256), (1024, 64, 272), (1000, 64, 1024), (256, 512, 768), (256, 512, 784), (250, 512, 1024),
+                                   (40, 384, 5472), (40, 448, 4096)])
+def test_rows_in_blocks_by_workgroups(M, K, N, epilogue):
+    """Both sides of the workgroup bounds of the 16-row blocks (three and four per compute unit)."""
+    rng = np.random.default_rng(M + K + N)
+    a, w, rq = _operands(rng, M, K, N, out_i8=False)
+    aux = rng.integers(-32768, 32768, (M, N)) if epilogue == "resadd" else None
+    got = gpu_linear(a, w, rq, out_i8=False, epilogue=epilogue, aux=aux)
+    assert np.array_equal(got, O.linear_c(a, w, rq, None, False, epilogue, aux, 0, None))
