@@ -624,18 +624,16 @@ __global__ __launch_bounds__(64 * AttnTileCfg<D>::MAXW, MINW) void attention_til
 #pragma unroll
       for (int c = 0; c < DK; ++c) vcache[it][j][c] = ld16(vr, kt < ntiles ? frag_off(kt, j, c) : LD_OOB);
   }
-  {
-    const Rsrc tr = rsrc(kExpT.v, sizeof(ExpTable));
-    for (int c = tid; c < EXPT_CHUNKS; c += 4 * (int)blockDim.x) {  // four chunks in flight per thread
-      v4i w[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) w[u] = ld16(tr, (uint32_t)(16 * (c + u * (int)blockDim.x)));
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (c + u * (int)blockDim.x < EXPT_CHUNKS) reinterpret_cast<v4i*>(tab)[c + u * (int)blockDim.x] = w[u];
-    }
-  }
   for (int idx = tid; idx < AT_ROWS * D; idx += blockDim.x) (&osum[0][0])[idx] = 0;
+  if (tid == 0) reinterpret_cast<v4i*>(tab)[EXPT_CHUNKS - 1] = v4i{0, 0, 0, 0};
+  // the table straight into LDS (1 KiB per wave and load, no registers, all in flight at once: staged
+  // through registers, four chunks per thread at a time, a launch of one wave per workgroup took 0.3 us
+  // more), but for its last chunk, the zeros from entry 4096 on
+  for (int b = wave; b < EXPT_CHUNKS / 64; b += nw) {
+    const int8_t* src = reinterpret_cast<const int8_t*>(kExpT.v) + b * 1024 + lane * 16;
+    int8_t* dst = reinterpret_cast<int8_t*>(tab) + b * 1024;
+    __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
+  }
   auto tile_max = [&](int kt, const v4i (&st)[4]) {
     if (kt < nfull) {
 #pragma unroll
@@ -666,6 +664,7 @@ __global__ __launch_bounds__(64 * AttnTileCfg<D>::MAXW, MINW) void attention_til
   vmax = max(vmax, __shfl_xor(vmax, 16));
   vmax = max(vmax, __shfl_xor(vmax, 32));
   if (lg == 0) red[wave][lr] = vmax;
+  __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's part of the table is in LDS
   __syncthreads();
   int32_t mx = red[0][lr];
   for (int w = 1; w < nw; ++w) mx = max(mx, red[w][lr]);
