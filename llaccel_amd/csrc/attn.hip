@@ -1631,25 +1631,31 @@ static int attention_impl(const int8_t* q, int64_t M, int64_t H, int64_t Hkv, in
   if (tiled) {
     // waves per workgroup: enough that every wave's tiles stay in registers across the three
     // passes, more (up to the register-file limit) while the chip would otherwise be idle.  Launches
-    // of at least one workgroup per CU stop at four waves while the rest of their tiles' packed
-    // probabilities take at most 32 KB of LDS (D >= 128, whose registers allow two or three waves
-    // per SIMD in any case: 64 KB): every wave repeats the prologue and the barriers.  Measured, four
-    // / eight waves: 1024 rows of D = 64 16.5 / 18.1 us, 8 x 1024 84.7 / 100 us, 1536 rows of D = 128
-    // 64.8 / 78.0 us, 4 x 512 40.8 / 63.8 us; past the limits 2048 rows of D = 64 48.4 / 41.2 us,
-    // 4096 rows of D = 128 512 / 435 us.
+    // of more than two workgroups per CU (D = 128: from one and a half on) stop at four waves while the rest of their
+    // tiles' packed probabilities take at most 32 KB of LDS (D = 128, whose registers allow one workgroup of
+    // eight waves or three of four per CU: 64 KB): every wave repeats the prologue and the barriers.
+    // Measured, the time with four waves over that with eight, by workgroups per CU: D = 16 to 64, 12 to
+    // 17 tiles: 1 1.17 to 1.25, 2 1.01 to 1.06, 2.25 0.82 to 0.96, 3 0.78 to 0.96, 5 0.93 to 1.0; D = 128, 8 to 19
+    // tiles: 1 1.11 to 1.17, 1.5 0.89 to 1.06, 2 0.86 to 0.99, 3 0.75 to 0.86 (1536 rows of 16 heads 64.8 / 78.0
+    // us); past the limits 2048 rows of D = 64 48.4 / 41.2 us, 4096 rows of D = 128 512 / 435 us.
     const int64_t blocks = H * ceil_div(M, AT_ROWS);
     const int maxw = D <= 128 ? AttnTileCfg<128>::MAXW : AttnTileCfg<256>::MAXW;
     const int sc = D <= 64 ? AttnTileCfg<64>::SC : 1;
     const int64_t tiles = ceil_div(tmax, 64);
-    const bool four = blocks >= cus && tiles <= 4 * (sc + (D <= 64 ? 4 : 8));
+    const bool four = (D <= 64 ? blocks > 2 * cus : 2 * blocks >= 3 * cus) && tiles <= 4 * (sc + (D <= 64 ? 4 : 8));
     int nw = 1;
     while (nw < (four ? std::min(maxw, 4) : maxw) && nw * 2 <= tiles && (nw * sc < tiles || blocks * nw < 4 * (int64_t)cus))
       nw *= 2;
     dim3 grid((unsigned)H, (unsigned)ceil_div(M, AT_ROWS));
     dim3 block(64 * nw);
-    // probabilities of the tiles past the cached ones kept in LDS: up to 64 KB, two workgroups per CU
+    // probabilities of the tiles past the cached ones kept in LDS: up to 64 KB, and where registers allow two
+    // workgroups per CU (D <= 64, or four waves of D = 128) no more than leaves both their static part as
+    // well (D = 128: the table, the output sums and the maxima, 16.5 KB; 2176 rows of 16 heads, 34 tiles: 158
+    // us with eight tiles' in LDS and one workgroup per CU, 118 with seven and the last computed again)
     const int64_t slots = std::max<int64_t>(0, ceil_div(tiles, nw) - sc);
-    p.pslots = (int)std::min<int64_t>(slots, (64 << 10) / (2048 * nw));
+    const int64_t fixed = (int64_t)sizeof(ExpTable) + 4 * AT_ROWS * (D + 8);
+    const int64_t room = D <= 64 || (D <= 128 && nw <= 4) ? std::min<int64_t>(64 << 10, (80 << 10) - fixed) : 64 << 10;
+    p.pslots = (int)std::min<int64_t>(slots, room / (2048 * nw));
     const unsigned lds = (unsigned)(p.pslots * nw * 2048);
     switch (D) {
       case 16: hipLaunchKernelGGL(attention_tiled<16>, grid, block, lds, s, p); break;

@@ -213,3 +213,12 @@ def test_softmax_regimes(M, D, regime):
         got = gpu_attention(q, kc, vc, pos, H, Hkv, D, Ms, Ss, Mo, So, pb)
         want = O.attention_c(q, kc, vc, pos, H, Hkv, D, Ms, Ss, Mo, So, pb)
         assert np.array_equal(got, want), pb
+
+
+@pytest.mark.parametrize("M,H,Hkv,D,pos,max_seq", [(520, 14, 2, 64, 500, 1024),    # eight waves, two workgroups per CU
+                                                   (600, 14, 2, 64, 400, 1024),    # four waves
+                                                   (384, 16, 8, 128, 1730, 2176),  # 34 tiles: seven in LDS, the last again
+                                                   (250, 24, 8, 128, 300, 640), (234, 24, 8, 128, 300, 640)])
+def test_waves_per_workgroup(M, H, Hkv, D, pos, max_seq):
+    """Both sides of the rule for four or eight waves, and four waves with more tiles than LDS keeps."""
+    test_attention_matches_oracle(M, H, Hkv, D, pos, max_seq)
