@@ -46,6 +46,9 @@ class FusedStep:
         self.K, self.bytes_fn, self.name, self.ops = K, bytes_fn, name, ops
         self.wide = wide_steps(model, ops, fallback)
         self.ffn = next(int(o["N"]) for o in ops if o.get("op") == "linear")  # mlp_in: its FFN columns
+        # what the fused kernel takes; weights are views into the qgraph's blob at its offsets, which need not be aligned
+        self.blocks_ok = kind == "mlp_in" and K % 16 == 0 and not any(
+            model._dt[t].data_ptr() % 16 for t in (ops[0]["gamma"], *(o["w"] for o in ops if o.get("op") == "linear")))
         self.lead = None  # a _LinearNormStep for the preceding resadd linear (see _pair_linear_norm)
 
     def in_blocks(self, M, pd=None):
@@ -54,7 +57,7 @@ class FusedStep:
         the tiled gate/up GEMM.  Prefill of 64 rows, 30 layers of 576 (FFN 1536) 1.47 -> 1.32 ms, 128
         rows 1.45 -> 1.38; 32 rows of 24 layers of 896 (FFN 4864) 1.10 -> 1.09, but 64 rows 1.14 ->
         1.17 ms.  (The attention run in blocks lost: 1.47 -> 1.74 ms at 64 rows of 576.)"""
-        if self.kind != "mlp_in" or not 16 < M <= 128 or 16 * (self.K + 16) > LDS_LIMIT or self.K > NORM_MAX_K:
+        if not self.blocks_ok or not 16 < M <= 128 or 16 * (self.K + 16) > LDS_LIMIT or self.K > NORM_MAX_K:
             return False
         return -(-M // 16) * self.ffn * self.K <= 12 << 20 and not _seq_rows(pd)
 

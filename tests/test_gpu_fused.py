@@ -349,3 +349,25 @@ def test_rows_normalised_without_quantised_rows_out():
     for a, b in zip(*outs):
         assert np.array_equal(a, b)
     assert np.abs(outs[0][2]).max() > 0
+
+
+def test_short_prompt_with_misaligned_mlp_weights(golden_dir, tmp_path):
+    """Weights at offsets that are no multiple of 16 bytes: a prompt of 17 to 128 rows is prefilled by the launches that
+    take them, as a longer one is."""
+    import json
+    import shutil
+
+    qdir = tmp_path / "q"
+    shutil.copytree(golden_dir / "ref_tiny_v2" / "qgraph", qdir)
+    prompt = list(range(2, 42))
+    want = np.stack(list(G.GoldenModel(qdir).prefill(prompt)))
+    q = json.loads((qdir / "qgraph.json").read_text())
+    gate = next(o for o in q["ops"] if o["op"] == "linear" and o.get("epilogue") == "silu")["w"]
+    blob = (qdir / q["weights_file"]).read_bytes()
+    spec = q["tensors"][gate]
+    data = blob[spec["offset"]:spec["offset"] + int(np.prod(spec["shape"]))]
+    blob += bytes(-len(blob) % 16 + 8)
+    spec["offset"] = len(blob)
+    (qdir / q["weights_file"]).write_bytes(blob + data)
+    (qdir / "qgraph.json").write_text(json.dumps(q))
+    assert np.array_equal(np.stack(list(G.GoldenModel(qdir).prefill(prompt))), want)
