@@ -23,6 +23,7 @@ import ctypes
 from . import _lib
 
 LDS_LIMIT = 48 * 1024
+CUS = 256  # compute units of the GPU
 NORM_MAX_K = 1024  # the fused RMSNorm prologue holds a row in two 8-element chunks per lane
 
 
@@ -45,21 +46,35 @@ class FusedStep:
         self.entry, self.desc = entry, desc_cls()
         self.K, self.bytes_fn, self.name, self.ops = K, bytes_fn, name, ops
         self.wide = wide_steps(model, ops, fallback)
-        self.ffn = next(int(o["N"]) for o in ops if o.get("op") == "linear")  # mlp_in: its FFN columns
-        # what the fused kernel takes; weights are views into the qgraph's blob at its offsets, which need not be aligned
-        self.blocks_ok = kind == "mlp_in" and K % 16 == 0 and not any(
-            model._dt[t].data_ptr() % 16 for t in (ops[0]["gamma"], *(o["w"] for o in ops if o.get("op") == "linear")))
+        self.blocks = self._blocks_limit() if kind == "mlp_in" else None
         self.lead = None  # a _LinearNormStep for the preceding resadd linear (see _pair_linear_norm)
 
+    def _blocks_limit(self):
+        """(FFN columns, largest number of 16-column x 16-row workgroups) for which a short prompt's MLP is run as
+        blocks of 16 rows of the fused kernel, or None: one launch in place of the norm and the tiled gate/up
+        GEMM, but the weights read again for every block.  Measured (us, blocks / norm and GEMM): FFN 1536 of
+        576, 64 rows 9.3 / 11.8, 96 rows 12.4 / 11.8 (384 and 576 workgroups); where K % 128 == 0 the GEMM has the
+        longer K tiles and the blocks win one per CU only: FFN 2048 of 768, 32 rows 8.1 / 8.5, 48 rows 9.6 / 8.7
+        (256 and 384); FFN 1024 of 1024, 64 rows 8.1 / 10.2; FFN 4864 of 896, 32 rows 9.75 / 9.0 (608); FFN 384 of 128,
+        32 rows 6.8 / 6.1 (a GEMM of few K tiles).  Without that GEMM (an unfused graph's separate ops, K not a multiple of 64) the
+        blocks win as long as re-reading the weights stays cheap: FFN 1000 of 592, 128 rows 9.8 / 320."""
+        lins = [o for o in self.ops if o.get("op") == "linear"]
+        N, K, dt = int(lins[0]["N"]), self.K, self.model._dt
+        # what the kernel takes; weights are views into the qgraph's blob at its offsets, which need not be aligned
+        if K % 16 or K > NORM_MAX_K or any(dt[t].data_ptr() % 16 for t in (self.ops[0]["gamma"], *(o["w"] for o in lins))):
+            return None
+        if K % 64 or not any(isinstance(st, _GateUpStep) for st in self.wide):
+            return N, (12 << 20) // (16 * K)  # 12 MiB per projection
+        if K % 128 == 0 and K < 384:
+            return None
+        return N, CUS if K % 128 == 0 else CUS * 3 // 2
+
     def in_blocks(self, M, pd=None):
-        """A short prompt's MLP run as blocks of 16 rows of the fused kernel: while reading the weights
-        again for every block stays cheap (12 MiB per projection), one launch in place of the norm and
-        the tiled gate/up GEMM.  Prefill of 64 rows, 30 layers of 576 (FFN 1536) 1.47 -> 1.32 ms, 128
-        rows 1.45 -> 1.38; 32 rows of 24 layers of 896 (FFN 4864) 1.10 -> 1.09, but 64 rows 1.14 ->
-        1.17 ms.  (The attention run in blocks lost: 1.47 -> 1.74 ms at 64 rows of 576.)"""
-        if not self.blocks_ok or not 16 < M <= 128 or 16 * (self.K + 16) > LDS_LIMIT or self.K > NORM_MAX_K:
+        """Whether M rows run as blocks of 16 rows of the fused kernel (see _blocks_limit)."""
+        if self.blocks is None or not 16 < M <= 128 or 16 * (self.K + 16) > LDS_LIMIT or _seq_rows(pd):
             return False
-        return -(-M // 16) * self.ffn * self.K <= 12 << 20 and not _seq_rows(pd)
+        N, most = self.blocks
+        return -(-M // 16) * -(-N // 16) <= most
 
     def takes_wide(self, M, pd=None):
         return (M > 16 or M * (self.K + 16) > LDS_LIMIT or self.K > NORM_MAX_K) and not self.in_blocks(M, pd)
