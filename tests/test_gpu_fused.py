@@ -371,3 +371,35 @@ def test_short_prompt_with_misaligned_mlp_weights(golden_dir, tmp_path):
     (qdir / q["weights_file"]).write_bytes(blob + data)
     (qdir / "qgraph.json").write_text(json.dumps(q))
     assert np.array_equal(np.stack(list(G.GoldenModel(qdir).prefill(prompt))), want)
+
+
+@pytest.mark.parametrize("fuse", [True, False])
+def test_prefill_rows_outlive_later_calls(golden_dir, fuse):
+    """The rows that prefill() returns stay what they are: those of an eager, a captured and a replayed prefill of one
+    length, read only after another prefill and a decode have run (with fuse=False the plan ends in a
+    linear of its own, whose rows are copied)."""
+    qdir = golden_dir / "ref_tiny_v2" / "qgraph"
+    g, e = G.GoldenModel(qdir, fuse=fuse), G.GoldenModel(qdir, fuse=fuse)
+    e.use_graph = False
+    assert (g._head_step(32) is not None) == fuse
+    prompts = [[(7 * i + 3 * j) % 60 for j in range(30)] for i in range(4)]
+    kept = []
+    for p in prompts:
+        g.reset()
+        kept.append(g.prefill(p))
+    g.decode(5, 30)
+    assert len(g._pf_graphs) == 1
+    for i, (p, rows) in enumerate(zip(prompts, kept)):
+        e.reset()
+        assert np.array_equal(rows.numpy(), np.stack(list(e.prefill(p)))), i
+
+
+def test_prefill_batch_rows_of_every_prompt(tmp_path_factory):
+    """Prompts of other lengths, each prefilled by itself: every prompt's rows, not the last one's alone."""
+    qdir = _qgraph(tmp_path_factory, "qwen25", True)
+    prompts = [synth.seeded_prompt("qwen25", n, n) for n in (40, 33, 47)]
+    rows = G.GoldenModel(qdir).prefill_batch(prompts)
+    s = G.GoldenModel(qdir)
+    for p, r in zip(prompts, rows):
+        s.reset()
+        assert np.array_equal(np.asarray(r[len(p) - 1]), np.asarray(s.prefill(p)[len(p) - 1]))
