@@ -188,7 +188,7 @@ def test_prefill_batch_other_lengths_run_separately(tmp_path_factory):
 @pytest.mark.parametrize("M", [2, 3, 4, 5, 7, 8, 9, 13, 16, 17, 33, 128])
 def test_rows_normalised_in_the_prologue(M, K, N):
     """llhip_mlp_in of several rows normalising them in every workgroup (several waves to a row, one
-    wave to one, two or more rows; past 8 rows and one workgroup per CU a launch of its own) writes
+    wave to one, two or more rows; from 8 rows on, past one workgroup per CU, a launch of its own) writes
     what llhip_rmsnorm_quant followed by the prequantised form writes."""
     import ctypes
 
