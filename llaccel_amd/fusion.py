@@ -54,10 +54,11 @@ class FusedStep:
         blocks of 16 rows of the fused kernel, or None: one launch in place of the norm and the tiled gate/up
         GEMM, but the weights read again for every block.  Measured (us, blocks / norm and GEMM): FFN 1536 of
         576, 64 rows 9.3 / 11.8, 96 rows 12.4 / 11.8 (384 and 576 workgroups); where K % 128 == 0 the GEMM has the
-        longer K tiles and the blocks win one per CU only: FFN 2048 of 768, 32 rows 8.1 / 8.5, 48 rows 9.6 / 8.7
-        (256 and 384); FFN 1024 of 1024, 64 rows 8.1 / 10.2; FFN 4864 of 896, 32 rows 9.75 / 9.0 (608); FFN 384 of 128,
-        32 rows 6.8 / 6.1 (a GEMM of few K tiles).  Without that GEMM (an unfused graph's separate ops, K not a multiple of 64) the
-        blocks win as long as re-reading the weights stays cheap: FFN 1000 of 592, 128 rows 9.8 / 320."""
+        longer K tiles and the blocks win up to one per CU only: FFN 2048 of 768, 32 rows 8.1 / 8.5, 48 rows 9.6 /
+        8.7 (256 and 384); FFN 1024 of 1024, 64 rows 8.1 / 10.2; FFN 4864 of 896, 32 rows 9.75 / 9.0 (608); FFN 384
+        of 128, 32 rows 6.8 / 6.1 (a GEMM of few K tiles).  Without that GEMM (an unfused graph's separate ops, K
+        not a multiple of 64) the blocks win as long as re-reading the weights stays cheap: FFN 1000 of 592, 128
+        rows 9.8 / 320."""
         lins = [o for o in self.ops if o.get("op") == "linear"]
         N, K, dt = int(lins[0]["N"]), self.K, self.model._dt
         # what the kernel takes; weights are views into the qgraph's blob at its offsets, which need not be aligned

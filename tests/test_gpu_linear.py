@@ -389,10 +389,11 @@ def test_partial_groups_of_loads(M, K, N, epilogue):
 
 
 @pytest.mark.parametrize("epilogue", ["none", "resadd"])
-@pytest.mark.parametrize("M,K,N", [(1024, 64, 256), (1024, 64, 272), (1000, 64, 1024), (256, 512, 768), (256, 512, 784), (250, 512, 1024),
-                                   (40, 384, 5472), (40, 448, 4096)])
+@pytest.mark.parametrize("M,K,N", [(1024, 64, 512), (1024, 64, 528), (1024, 64, 640), (1024, 64, 656), (256, 512, 1040), (256, 512, 1056),
+                                   (250, 512, 1456), (250, 512, 1472), (40, 384, 8768), (40, 384, 8784), (32, 192, 24000)])
 def test_rows_in_blocks_by_workgroups(M, K, N, epilogue):
-    """Both sides of the workgroup bounds of the 16-row blocks (three and four per compute unit)."""
+    """Both sides of the workgroup bounds of the 16-row blocks: K % 64 == 0 (eight per compute unit, ten with an epilogue),
+    K % 128 == 0 (by K), and more where the last 64 rows of a tile are partly empty."""
     rng = np.random.default_rng(M + K + N)
     a, w, rq = _operands(rng, M, K, N, out_i8=False)
     aux = rng.integers(-32768, 32768, (M, N)) if epilogue == "resadd" else None
